@@ -29,58 +29,67 @@ struct RawBlk {
   u32x4_t q0, q1, h;
 };
 
-// qrow / hrow: the row's payload and header planes; b: the block
-template <int TYPE>
-__device__ __forceinline__ RawBlk load_block_at(const uint8_t* qrow, const uint8_t* hrow, int b) {
-  using Tr = Traits<TYPE>;
-  const uint8_t* qp = qrow + (uint32_t)(b * Tr::QB);
-  const uint8_t* hp = hrow + (uint32_t)((b >> 3) * Tr::HB);
+template <bool STREAM>
+__device__ __forceinline__ u32x4_t ld16(const void* p) {
+  if constexpr (STREAM) return ld_stream16(p);
+  else return *(const u32x4_t*)p;
+}
+template <bool STREAM>
+__device__ __forceinline__ uint32_t ld4(const uint32_t* p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
+// qp / hp: the block's payload record and its superblock's header record; ib: the block's index in the superblock
+// STREAM: non-temporal payload loads, where one lane group reads whole lines (a line shared with other waves stays)
+template <int TYPE, bool STREAM = true>
+__device__ __forceinline__ RawBlk load_block_ptr(const uint8_t* qp, const uint8_t* hp, int ib) {
   RawBlk r;
   r.q1 = u32x4_t{0u, 0u, 0u, 0u};
   r.h = u32x4_t{0u, 0u, 0u, 0u};
   if constexpr (TYPE == T_Q8_0) {
-    r.q0 = ld_stream16(qp);
-    r.q1 = ld_stream16(qp + 16);
-    r.h.x = ((const uint16_t*)hp)[b & 7];
+    r.q0 = ld16<STREAM>(qp);
+    r.q1 = ld16<STREAM>(qp + 16);
+    r.h.x = ((const uint16_t*)hp)[ib];
   } else if constexpr (TYPE == T_Q4_0 || TYPE == T_IQ4_NL) {
-    r.q0 = ld_stream16(qp);
-    r.h.x = ((const uint16_t*)hp)[b & 7];
+    r.q0 = ld16<STREAM>(qp);
+    r.h.x = ((const uint16_t*)hp)[ib];
   } else if constexpr (kIq1<TYPE>) {
     const uint32_t* q = (const uint32_t*)qp;
-    r.q0 = u32x4_t{__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1), 0u, 0u};
+    r.q0 = u32x4_t{ld4<STREAM>(q), ld4<STREAM>(q + 1), 0u, 0u};
     r.h.x = *(const uint32_t*)hp;  // f16 d
   } else if constexpr (TYPE == T_Q2_0 || TYPE == T_Q2_K) {
     const uint32_t* q = (const uint32_t*)qp;
-    r.q0 = u32x4_t{__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1), 0u, 0u};
+    r.q0 = u32x4_t{ld4<STREAM>(q), ld4<STREAM>(q + 1), 0u, 0u};
     if constexpr (TYPE == T_Q2_0) {
-      r.h.x = ((const uint16_t*)hp)[block_scale_slot<TYPE>(b & 7)];
+      r.h.x = ((const uint16_t*)hp)[block_scale_slot<TYPE>(ib)];
     } else {
       r.h.x = *(const uint32_t*)hp;                  // d, dmin
-      r.h.y = ((const uint16_t*)(hp + 4))[b & 7];   // the block's two scale / min bytes
+      r.h.y = ((const uint16_t*)(hp + 4))[ib];   // the block's two scale / min bytes
     }
   } else if constexpr (TYPE == T_Q3_K) {
     const uint32_t* q = (const uint32_t*)qp;
-    r.q0 = u32x4_t{__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1), __builtin_nontemporal_load(q + 2),
+    r.q0 = u32x4_t{ld4<STREAM>(q), ld4<STREAM>(q + 1), ld4<STREAM>(q + 2),
                    0u};
-    r.h.x = ((const uint16_t*)hp)[b & 7];  // the block's two int8 scales
+    r.h.x = ((const uint16_t*)hp)[ib];  // the block's two int8 scales
     r.h.y = ((const uint16_t*)hp)[8];      // f16 d
   } else if constexpr (TYPE == T_Q5_K) {
-    r.q0 = ld_stream16(qp);
-    r.q1.x = __builtin_nontemporal_load((const uint32_t*)(qp + 16));
+    r.q0 = ld16<STREAM>(qp);
+    r.q1.x = ld4<STREAM>((const uint32_t*)(qp + 16));
     r.h = *(const u32x4_t*)hp;
   } else if constexpr (TYPE == T_Q6_K) {
-    r.q0 = ld_stream16(qp);
+    r.q0 = ld16<STREAM>(qp);
     const uint32_t* q = (const uint32_t*)(qp + 16);
-    r.q1.x = __builtin_nontemporal_load(q);
-    r.q1.y = __builtin_nontemporal_load(q + 1);
-    r.h.x = ((const uint16_t*)hp)[b & 7];  // the block's two int8 scales
+    r.q1.x = ld4<STREAM>(q);
+    r.q1.y = ld4<STREAM>(q + 1);
+    r.h.x = ((const uint16_t*)hp)[ib];  // the block's two int8 scales
     r.h.y = ((const uint16_t*)hp)[8];      // f16 d
   } else if constexpr (kIq2<TYPE>) {
     // (payload words q0.x..z; header: IQ2_XS scales in h.x, h.y and d in h.z, IQ2_S qh in h.x, h.y, scales in
     //  h.z, h.w and d in q1.x, the others d in h.x)
     const uint32_t* q = (const uint32_t*)qp;
-    r.q0 = u32x4_t{__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1),
-                   TYPE == T_IQ3_XXS ? __builtin_nontemporal_load(q + 2) : 0u, 0u};
+    r.q0 = u32x4_t{ld4<STREAM>(q), ld4<STREAM>(q + 1),
+                   TYPE == T_IQ3_XXS ? ld4<STREAM>(q + 2) : 0u, 0u};
     const uint32_t* hw = (const uint32_t*)hp;
     if constexpr (TYPE == T_IQ2_XS) {
       r.h.x = hw[0];
@@ -94,11 +103,11 @@ __device__ __forceinline__ RawBlk load_block_at(const uint8_t* qrow, const uint8
     }
   } else if constexpr (TYPE == T_IQ3_S) {
     const uint32_t* q = (const uint32_t*)qp;
-    r.q0 = u32x4_t{__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1), __builtin_nontemporal_load(q + 2),
+    r.q0 = u32x4_t{ld4<STREAM>(q), ld4<STREAM>(q + 1), ld4<STREAM>(q + 2),
                    0u};
     r.h = *(const u32x4_t*)hp;
   } else {
-    r.q0 = ld_stream16(qp);
+    r.q0 = ld16<STREAM>(qp);
     if constexpr (TYPE == T_IQ4_XS) {
       const uint2 h = *(const uint2*)hp;
       r.h.x = h.x;
@@ -108,6 +117,13 @@ __device__ __forceinline__ RawBlk load_block_at(const uint8_t* qrow, const uint8
     }
   }
   return r;
+}
+
+// qrow / hrow: the row's payload and header planes; b: the block
+template <int TYPE>
+__device__ __forceinline__ RawBlk load_block_at(const uint8_t* qrow, const uint8_t* hrow, int b) {
+  using Tr = Traits<TYPE>;
+  return load_block_ptr<TYPE>(qrow + (uint32_t)(b * Tr::QB), hrow + (uint32_t)((b >> 3) * Tr::HB), b & 7);
 }
 
 template <int TYPE>

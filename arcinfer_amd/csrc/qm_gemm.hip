@@ -1058,10 +1058,10 @@ static hipError_t dispatch(int mode, const GemmArgs& a, hipStream_t s) {
 
 template <int TYPE>
 static hipError_t dispatch_s16(int mode, const GemmArgs& a, hipStream_t s) {
-  if (a.dbg_isum) return a.M <= 32 ? go_s16<TYPE, 1, GEMM_DENSE, true>(a, s) : go_s16<TYPE, 2, GEMM_DENSE, true>(a, s);
+  if (a.dbg_isum) return go_s16<TYPE, 2, GEMM_DENSE, true>(a, s);
   switch (mode) {
     case GEMM_DENSE:
-      return a.M <= 32 ? go_s16<TYPE, 1, GEMM_DENSE, false>(a, s) : go_s16<TYPE, 2, GEMM_DENSE, false>(a, s);
+      return go_s16<TYPE, 2, GEMM_DENSE, false>(a, s);  // (up to 32 tokens: the few-token kernels)
     // (MoE modes over slot-tile pairs: at the BASELINE MoE shape Q6_K down 0.94 -> 0.82 ms for the layer, all-Q6_K
     //  1.50 -> 1.16, IQ2_XS unchanged)
     case GEMM_MOE_G: return go_s16<TYPE, 2, GEMM_MOE_G, false>(a, s);
@@ -1072,6 +1072,9 @@ static hipError_t dispatch_s16(int mode, const GemmArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s) {
+  if (mode == GEMM_DENSE && skinny_supported(type, true, a.M, a.w.rows, a.w.K))
+    return launch_skinny(type, SkinnyArgs{a.w, a.aq, a.asc, a.absum, a.M, a.M_stride, a.ash, a.C, a.ldc, a.c_off, a.accumulate,
+                                          a.dbg_isum, nullptr}, s);
   switch (type) {
     case T_Q6_K: return dispatch_s16<T_Q6_K>(mode, a, s);
     case T_Q3_K: return dispatch_s16<T_Q3_K>(mode, a, s);

@@ -6,6 +6,9 @@ namespace qm {
 template <int TYPE> hipError_t gemv_dispatch(const GemvArgs& a, hipStream_t s);
 
 hipError_t launch_gemv(int type, const GemvArgs& a, hipStream_t s) {
+  if (skinny_supported(type, false, a.T, a.w.rows, a.w.K))
+    return launch_skinny(type, SkinnyArgs{a.w, a.aq, a.asc, a.absum, a.T, a.M_stride, 0, a.C, a.ldc, a.c_off, a.accumulate,
+                                          a.dbg_isum, a.dbg_msum}, s);
   switch (type) {
     case T_Q8_0: return gemv_dispatch<T_Q8_0>(a, s);
     case T_Q4_K: return gemv_dispatch<T_Q4_K>(a, s);

@@ -1,4 +1,5 @@
-// Decode GEMV on the prepared planes: C[t][n] (+)= sum_k W[n][k] * a_t[k] for T <= 8 tokens per weight read.
+// Decode GEMV on the prepared planes: C[t][n] (+)= sum_k W[n][k] * a_t[k] for T <= 4 tokens per weight read (more tokens, and
+// three or four where they are faster, go to the few-token kernels, qm_skinny_impl.h).
 //
 // Mapping: a wave is split into 64/LPR lane groups; each group owns R consecutive rows and walks the row's 32-blocks
 // with its LPR lanes (lane j: blocks j, j + LPR, ...). Per block a lane loads the token activations once (32 int8 +
@@ -276,9 +277,6 @@ __global__ __launch_bounds__(NT) void gemvs_kernel(GemvArgs a) {
           }
         }
       }
-      // (eight tokens: one block's token rows at a time -- left free, the compiler reads every block's rows for
-      // every token from LDS up front and runs out of registers)
-      if constexpr (TB >= 8) __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (PF == 2 && !EXACT) {
       // (the last chunk is decoded under a branch that whole waves skip; a use of its registers on every path marks
@@ -352,12 +350,6 @@ __global__ __launch_bounds__(NT) void gemvs_kernel(GemvArgs a) {
   }
 }
 
-// Most tokens per gemvs_kernel launch: 8, or 4 where eight tokens' registers would spill (more than 5 blocks per lane,
-// more than 4 for Q6_K) or where two 4-token launches measured faster (IQ2_XXS at 4+ blocks per lane, applied to the
-// grid-decoded types alike); more tokens run as chunks.
-template <int TYPE>
-constexpr int gemvs_max_tb(int ch) { return ch <= (TYPE == T_Q6_K ? 4 : (kIq2<TYPE> || kIq1<TYPE>) ? 3 : 5) ? 8 : 4; }
-
 // LDS bytes of gemvs_kernel for TB tokens (the per-16 sums for the types that read them: kNeedsBsum)
 template <int TYPE>
 static size_t gemvs_lds(int K, int TB) {
@@ -375,8 +367,7 @@ static hipError_t gos(const GemvArgs& a0, hipStream_t s) {
   // 17.7 -> 21.6 us)
   constexpr int PF = TB == 1 || (TB == 2 && CH <= 5) ? 2 : 1;
   // Persistent grid: PC work-groups per CU (two; three with four waves per row or where measured faster), or as many
-  // as the kernel's registers and LDS let reside (the 8-token instantiation needs more than 256 registers: one wave per
-  // SIMD), so the whole grid is resident at once; fewer when the matrix has fewer rows than lane groups. Occupancy is
+  // as the kernel's registers and LDS let reside, so the whole grid is resident at once; fewer when the matrix has fewer rows than lane groups. Occupancy is
   // queried once, for this instantiation's largest K.
   static const int per_cu = [] {
     int n = 0;
@@ -402,7 +393,7 @@ static hipError_t gos(const GemvArgs& a0, hipStream_t s) {
 
 template <int TYPE, int LPR, int CH, bool EXACT, bool DUMP>
 static hipError_t gos_tb(const GemvArgs& a, hipStream_t s) {
-  switch (a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8) {
+  switch (a.T <= 1 ? 1 : a.T <= 2 ? 2 : 4) {
     case 1:
       // batch 1, 32 lanes per row (K 5120 -> N 17408, A/B in one process): IQ3_S and IQ3_XXS with the token blocks in
       // registers and three work-groups per CU 14.0 -> 13.1 and 12.5 -> 12.0 us (less LDS traffic beside their
@@ -411,10 +402,9 @@ static hipError_t gos_tb(const GemvArgs& a, hipStream_t s) {
       if constexpr (LPR == 32 && TYPE == T_Q3_K) return gos<TYPE, LPR, CH, EXACT, 1, DUMP, false, 3>(a, s);
       return gos<TYPE, LPR, CH, EXACT, 1, DUMP>(a, s);
     case 2: return gos<TYPE, LPR, CH, EXACT, 2, DUMP>(a, s);
-    case 4: return gos<TYPE, LPR, CH, EXACT, 4, DUMP>(a, s);
     default:
-      if constexpr (gemvs_max_tb<TYPE>(CH) >= 8) return gos<TYPE, LPR, CH, EXACT, 8, DUMP>(a, s);
-      else return hipErrorInvalidValue;  // (the dispatcher never asks: it chunks by gemvs_max_tb)
+      if constexpr (LPR * CH <= 512) return gos<TYPE, LPR, CH, EXACT, 4, DUMP>(a, s);
+      else return hipErrorInvalidValue;  // (rows past 512 blocks: three tokens and more go to the few-token kernels)
   }
 }
 
@@ -434,9 +424,9 @@ static hipError_t gemv_route(const GemvArgs& a, hipStream_t s) {
   const int nb = a.w.K / 32;
   const bool l32 = nb % 32 == 0;
   if (nb <= 1024) {
-    // tokens per launch: as many as fit in 80 KB of LDS (two work-groups per CU), up to 8; more tokens -> chunks
+    // tokens per launch: as many as fit in 80 KB of LDS (two work-groups per CU), up to 4; more tokens -> chunks
     // of tokens, each launch reading the weights once
-    int tb = gemvs_max_tb<TYPE>(nb <= 256 ? (nb + 31) / 32 : (nb + 127) / 128);
+    int tb = nb <= 512 ? 4 : 2;
     const size_t cap = 80 * 1024 - sizeof(typename LdsFor<TYPE>::type);  // (the codebook tables' static LDS)
     while (tb > 1 && gemvs_lds<TYPE>(a.w.K, tb) > cap) tb >>= 1;
     for (int t0 = 0; t0 < a.T; t0 += tb) {
@@ -500,9 +490,7 @@ static hipError_t gemv_route(const GemvArgs& a, hipStream_t s) {
     // long rows (K > 32768: few rows): one row per lane group, for more waves in flight
     return l32 ? go<TYPE, 32, 1, 1, DUMP>(a, s) : go<TYPE, 8, 2, 1, DUMP>(a, s);
   }
-  if (a.T <= 2) return l32 ? go<TYPE, 32, 1, 2, DUMP>(a, s) : go<TYPE, 8, 1, 2, DUMP>(a, s);
-  if (a.T <= 4) return l32 ? go<TYPE, 32, 1, 4, DUMP>(a, s) : go<TYPE, 8, 1, 4, DUMP>(a, s);
-  return l32 ? go<TYPE, 32, 1, 8, DUMP>(a, s) : go<TYPE, 8, 1, 8, DUMP>(a, s);
+  return l32 ? go<TYPE, 32, 1, 2, DUMP>(a, s) : go<TYPE, 8, 1, 2, DUMP>(a, s);
 }
 
 template <int TYPE>

@@ -31,6 +31,25 @@ struct GemvArgs {
 };
 hipError_t launch_gemv(int type, const GemvArgs& a, hipStream_t s);
 
+// Products of 1 to 32 tokens against one read of the weight on the int8 matrix pipe (qm_skinny_*.hip). Any weight type,
+// rows and K; dbg_isum: block-sum mode.
+struct SkinnyArgs {
+  WView w;
+  const int8_t* aq;
+  const float* asc;
+  const int16_t* absum;
+  int M, M_stride;
+  int ash;  // asc row of 32-block b: b >> ash
+  float* C;
+  int ldc, c_off, accumulate;
+  int32_t* dbg_isum;
+  int32_t* dbg_msum;
+};
+constexpr int kSkinnyMax = 32;
+// whether a decode GEMV (prompt = false) or prompt GEMM of M tokens goes there
+bool skinny_supported(int type, bool prompt, int M, int rows, int K);
+hipError_t launch_skinny(int type, const SkinnyArgs& a, hipStream_t s);
+
 // Row source of a GEMM's activation tile: dense (row m = token m), gathered (row r = token rowmap[r]) or slots.
 struct GemmArgs {
   WView w;       // weight (MoE: gate or down, stacked experts)
