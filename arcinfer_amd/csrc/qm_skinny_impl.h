@@ -428,7 +428,7 @@ static hipError_t skinny_route(const SkinnyArgs& a, hipStream_t s) {
 
 // Which calls the few-token kernels take. Decode (T <= 8): from 5 tokens on always (1.2-3.3 x the GEMV's time before). 3 and
 // 4 tokens: rows past 16384, where the GEMV splits its tokens over launches (5120 x 17408: IQ4_XS 41.9 -> 22.4 us, Q4_K 34.8 ->
-// 25.8, Q8_0 37.7 -> 34.0; Q2_K, with mins per 16, only at four: 33.9 -> 30.9, at three 28.4 against 30.9), and the types of 16-byte records up to 8192 rows of at most 5120 (4096 x 4096: 7.3 -> 5.5 us; the
+// 25.8, Q8_0 37.7 -> 34.0; Q2_K, with mins per 16, only at four: 33.9 -> 30.9, at three 28.4 against 30.9; past 32768 the GEMV takes two tokens at most), and the types of 16-byte records up to 8192 rows of at most 5120 (4096 x 4096: 7.3 -> 5.5 us; the
 // others' heavier decode leaves them level or behind: Q8_0 512 x 5120 6.6 against 7.1, Q6_K 1024 x 1024 3.6 against 3.75).
 // Prompts: up to 16 tokens always (1.2-5.7 x); 17 to 32 unless the matrix is too large for one-tile work-groups to fit the
 // chip in a round or two and its rows too long for the sweep (17408 x 8192: IQ4_XS 54.5 against 63.0 us; Q6_K 89.6 against 84.7,
@@ -437,7 +437,7 @@ template <int TYPE>
 bool skinny_takes(bool prompt, int M, int rows, int K) {
   if (M > kSkinnyMax || M < 3) return prompt && M < 3;
   if (prompt) return M <= 16 || kHalves<TYPE> || rows <= 8192 || skinny_sweeps<TYPE>(M, rows, K);
-  return M >= 5 || (K > 16384 && (M == 4 || !kMin16<TYPE>)) || (Traits<TYPE>::QB == 16 && rows <= 8192 && K <= 5120);
+  return M >= 5 || (K > 16384 && (M == 4 || K > 32768 || !kMin16<TYPE>)) || (Traits<TYPE>::QB == 16 && rows <= 8192 && K <= 5120);
 }
 
 template <int TYPE>
