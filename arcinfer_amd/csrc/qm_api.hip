@@ -427,26 +427,56 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   a.accumulate = accumulate;
   a.ash = act32 ? 0 : 3;
   hipError_t e;
-  if (qm::f16_gemm_supported(w->type, M, w->view.K)) {
-    void* scr = nullptr;  // null: the f16 path takes its workspace from the per-device pool
-    const size_t need = qm::f16_workspace_bytes(M, w->view.K);
-    if (wm == WS_STATIC) {
-      size_t cap = 0;
-      e = qm::f16_scratch(&scr, &cap);
-      if (e != hipSuccess) return hip_fail(e, "qmatmul_gemm_noalloc: scratch lookup");
-      if (need > cap)
-        return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs %zu bytes of scratch, the static scratch holds %zu "
-                    "(use qmatmul_gemm or qmatmul_gemm_ws)", fn, M, w->view.K, need, cap);
-    } else if (wm == WS_CALLER) {
-      if (!ws || ws_bytes < need)
+  const bool f16 = qm::f16_gemm_supported(w->type, M, w->view.K);
+  const size_t need = f16 ? align256(qm::f16_workspace_bytes(M, w->view.K)) : 0;  // the f16 path's activations
+  const qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, w->view.K);
+  const size_t pb = sp.splits > 1 ? sp.bytes : 0;                                 // partial tiles (optional)
+  void *scr = nullptr, *pool = nullptr;
+  float* part = nullptr;
+  if (wm == WS_STATIC) {
+    size_t cap = 0;
+    void* ps = nullptr;
+    e = qm::f16_scratch(&scr, &cap, &ps);
+    if (e != hipSuccess) return hip_fail(e, "qmatmul_gemm_noalloc: scratch lookup");
+    if (f16 && qm::f16_workspace_bytes(M, w->view.K) > cap)
+      return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs %zu bytes of scratch, the static scratch holds %zu "
+                  "(use qmatmul_gemm or qmatmul_gemm_ws)", fn, M, w->view.K, need, cap);
+    if (pb) part = (float*)ps;
+  } else if (wm == WS_CALLER) {
+    if (f16) {
+      if (!ws || ws_bytes < qm::f16_workspace_bytes(M, w->view.K))
         return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs a workspace of %zu bytes (given %zu%s)", fn, M,
                     w->view.K, need, ws_bytes, ws ? "" : ", null");
       if (!aligned(ws, 256)) return fail(QM_ERR_ARG, "%s: the workspace must be 256-byte aligned", fn);
       scr = ws;
     }
-    e = qm::launch_gemm_f16(w->type, a, scr, (hipStream_t)stream);
-  } else {
-    e = qm::launch_gemm(w->type, qm::GEMM_DENSE, a, (hipStream_t)stream);  // (this kernel uses no workspace)
+    if (pb && ws && ws_bytes >= need + pb && aligned(ws, 256)) part = (float*)((uint8_t*)ws + need);
+  } else if (f16 || pb) {
+    // (a capturing stream: no partial tiles, so the types that need no workspace record no allocation)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const bool cut = pb && hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+    if (need || cut) {
+      e = qm::pool_alloc(&pool, need + (cut ? pb : 0), (hipStream_t)stream);
+      if (e != hipSuccess && f16) return hip_fail(e, fn);
+      if (e == hipSuccess) {
+        scr = pool;
+        if (cut) part = (float*)((uint8_t*)pool + need);
+      } else {
+        pool = nullptr;
+        (void)hipGetLastError();  // (no partial tiles then: the uncut kernels need no memory)
+      }
+    }
+  }
+  if (part) {
+    a.part = part;
+    a.split_from = sp.from;
+    a.splits = sp.splits;
+  }
+  e = f16 ? qm::launch_gemm_f16(w->type, a, scr, (hipStream_t)stream)
+          : qm::launch_gemm(w->type, qm::GEMM_DENSE, a, (hipStream_t)stream);
+  if (pool) {
+    const hipError_t e2 = hipFreeAsync(pool, (hipStream_t)stream);
+    if (e == hipSuccess) e = e2;
   }
   return e == hipSuccess ? QM_OK : hip_fail(e, fn);
 }
@@ -465,7 +495,9 @@ int qmatmul_gemm_ex(const qm_weight* w, const int8_t* aq, const float* asc, cons
 
 size_t qmatmul_gemm_workspace_size(const qm_weight* w, int M) {
   if (!w || M < 1) return 0;
-  return qm::f16_gemm_supported(w->type, M, w->view.K) ? qm::f16_workspace_bytes(M, w->view.K) : 0;
+  const size_t need = qm::f16_gemm_supported(w->type, M, w->view.K) ? qm::f16_workspace_bytes(M, w->view.K) : 0;
+  const qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, w->view.K);
+  return sp.splits > 1 ? align256(need) + sp.bytes : need;
 }
 
 int qmatmul_gemm_ws(const qm_weight* w, const int8_t* aq, const float* asc, const int16_t* absum, int M, int M_stride,

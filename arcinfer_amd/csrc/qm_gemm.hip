@@ -23,6 +23,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int A_STRIDE = 272;  // LDS bytes per staged activation row
 
@@ -199,15 +200,23 @@ __device__ __forceinline__ void sb_scales(uint4 h, const uint4* pay, float dsc[8
   }
 }
 
-// Work-group -> (column tile, row tile). Dense launches are remapped so that each of the 8 XCDs (work-groups are
+// Work-group -> (column tile, row tile, K piece). The whole tiles are remapped so that each of the 8 XCDs (work-groups are
 // dealt to XCDs round-robin) sweeps a contiguous range of column tiles, row tiles fastest: concurrent work-groups
-// of an XCD share weight tiles in its L2.
-__device__ __forceinline__ void dense_tile(int& nt, int& mtile) {
-  const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
-  int lin = blockIdx.y * gx + blockIdx.x;
-  if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
+// of an XCD share weight tiles in its L2. Returns the index of the piece among the cut tiles' pieces, or -1 for a whole tile.
+template <bool CUT>
+__device__ __forceinline__ int dense_tile(const GemmArgs& a, int bm, int& nt, int& mtile) {
+  const int gy = (a.M + bm - 1) / bm;
+  int lin = blockIdx.x, piece = -1;
+  const int whole = CUT ? a.split_from : (int)gridDim.x;
+  if (CUT && lin >= whole) {
+    piece = lin - whole;
+    lin = whole + piece / a.splits;
+  } else if (whole % 8 == 0) {
+    lin = (lin % 8) * (whole / 8) + lin / 8;
+  }
   nt = lin / gy;
   mtile = lin % gy;
+  return piece;
 }
 
 // lo in lanes where m is 0, hi where m is all ones
@@ -251,11 +260,12 @@ __device__ __forceinline__ void moe_store(const GemmArgs& a, int slot, int n, bo
 // The work-group's rows: a dense M tile, or (MoE modes) one sub-tile of BM slots of an expert's tile of up to
 // kMoeTileRows slots (returns false for work-groups past the tile count or past the tile's rows). wrow0: the
 // expert's first weight row.
-template <int MODE, int BM>
-__device__ __forceinline__ bool tile_rows(const GemmArgs& a, int& m0, int& nvalid, int& wrow0, int& nt) {
+template <int MODE, int BM, bool CUT>
+__device__ __forceinline__ bool tile_rows(const GemmArgs& a, int& m0, int& nvalid, int& wrow0, int& nt, int& piece) {
+  piece = -1;
   if constexpr (MODE == GEMM_DENSE) {
     int mtile;
-    dense_tile(nt, mtile);
+    piece = dense_tile<CUT>(a, BM, nt, mtile);
     m0 = mtile * BM;
     nvalid = min(BM, a.M - m0);
     wrow0 = 0;
@@ -286,7 +296,18 @@ __device__ __forceinline__ bool tile_rows(const GemmArgs& a, int& m0, int& nvali
   }
 }
 
-template <int TYPE, int MT, int MODE, bool DUMP>
+// A cut tile's partial sums: piece-local [32 MT rows][128 columns]
+template <int MT>
+__device__ __forceinline__ void store_piece(const GemmArgs& a, int piece, int wave, int hf, int lc, const v16f* acc) {
+  float* p = a.part + (size_t)piece * (32 * MT * 128) + wave * 32 + lc;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[(mt * 32 + 8 * (r >> 2) + 4 * hf + (r & 3)) * 128] = acc[mt][r];
+}
+
+// CUT: the launch has pieces of cut tiles (a.part)
+template <int TYPE, int MT, int MODE, bool DUMP, bool CUT = false>
 __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
   constexpr int BM = 32 * MT;
   constexpr bool MINS = Traits<TYPE>::MINS;
@@ -296,12 +317,14 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
   __shared__ GemmLds<TYPE, MT> L;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hf = lane >> 5, lc = lane & 31;
   const int K = a.w.K, nb = K / 32, nsb = K / 256;
-  // K split (dense, gridDim.z = 2): this work-group's superblocks [sb0, sb1); the two halves are added into a zeroed C
-  const int sb0 = (int)blockIdx.z * nsb / (int)gridDim.z, sb1 = ((int)blockIdx.z + 1) * nsb / (int)gridDim.z;
-
   // ---- which rows: dense (M tile), or one MoE tile (expert e, slots r0 .. r0 + nr - 1)
-  int m0, nvalid, wrow0, nt;
-  if (!tile_rows<MODE, BM>(a, m0, nvalid, wrow0, nt)) return;
+  int m0, nvalid, wrow0, nt, piece;
+  if (!tile_rows<MODE, BM, CUT>(a, m0, nvalid, wrow0, nt, piece)) return;
+  // this work-group's superblocks [sb0, sb1): its piece of a cut tile, or one of the two halves that are added into a zeroed C
+  // (gridDim.z = 2)
+  const int z = !CUT ? (int)blockIdx.z : piece >= 0 ? piece % a.splits : 0;
+  const int nz = !CUT ? (int)gridDim.z : piece >= 0 ? a.splits : 1;
+  const int sb0 = z * nsb / nz, sb1 = (z + 1) * nsb / nz;
   const int n_loc = nt * 128 + wave * 32 + lc;  // this lane's weight row (within the expert)
   const int n_rows = MODE == GEMM_DENSE ? a.w.rows : a.expert_rows;
   const int n = wrow0 + min(n_loc, n_rows - 1);
@@ -579,6 +602,10 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
 
   // ---- epilogue
   const bool col_ok = n_loc < n_rows;
+  if (CUT && piece >= 0) {
+    store_piece<MT>(a, piece, wave, hf, lc, acc);
+    return;
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
@@ -615,7 +642,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
 // signed int8 (Q6_K: the 6-bit value minus 32, a byte-wise subtract without borrows; IQ2: grid words with their
 // signs, groups h and 2 + h of the block); one 2-block f32 outer product gives asc * d * sc for both halves (lanes
 // 0-31: the first half's scale, lanes 32-63: the second's). Tiles, staging and epilogue as gemm_kernel's dense mode.
-template <int TYPE, int MT, int MODE, bool DUMP>
+template <int TYPE, int MT, int MODE, bool DUMP, bool CUT = false>
 __global__ __launch_bounds__(256, 2) void gemm_s16_kernel(GemmArgs a) {
   constexpr int BM = 32 * MT;
   constexpr int ACH = BM * 16 / 256;
@@ -624,8 +651,10 @@ __global__ __launch_bounds__(256, 2) void gemm_s16_kernel(GemmArgs a) {
   __shared__ GemmLds<TYPE, MT> L;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hf = lane >> 5, lc = lane & 31;
   const int K = a.w.K, nb = K / 32, nsb = K / 256;
-  int m0, nvalid, wrow0, nt;
-  if (!tile_rows<MODE, BM>(a, m0, nvalid, wrow0, nt)) return;
+  int m0, nvalid, wrow0, nt, piece;
+  if (!tile_rows<MODE, BM, CUT>(a, m0, nvalid, wrow0, nt, piece)) return;
+  const int z = CUT && piece >= 0 ? piece % a.splits : 0, nz = CUT && piece >= 0 ? a.splits : 1;
+  const int sb0 = z * nsb / nz, sb1 = (z + 1) * nsb / nz;  // (its piece of a cut tile, or all superblocks)
   const int n_loc = nt * 128 + wave * 32 + lc;
   const int n_rows = MODE == GEMM_DENSE ? a.w.rows : a.expert_rows;
   const int n = wrow0 + min(n_loc, n_rows - 1);
@@ -689,7 +718,7 @@ __global__ __launch_bounds__(256, 2) void gemm_s16_kernel(GemmArgs a) {
   };
   uint2 nib[8], hw[8];
 #pragma unroll
-  for (int b = 0; b < 8; ++b) load_blk(b, nib[b], hw[b]);
+  for (int b = 0; b < 8; ++b) load_blk(sb0 * 8 + b, nib[b], hw[b]);
   // (header records are 20 or 12 bytes: 4-byte aligned, so read as dwords) sc: Q6_K / Q3_K int8 scales[16], IQ2_XS
   // scales[8] (.x .y), IQ2_S qh[8] (.x .y) and scales[8] (.z .w); dd: f16 d
   auto load_hdr = [&](int sb, uint4& sc, uint32_t& dd) {
@@ -710,7 +739,7 @@ __global__ __launch_bounds__(256, 2) void gemm_s16_kernel(GemmArgs a) {
   };
   uint4 hsc;
   uint32_t hd;
-  load_hdr(0, hsc, hd);
+  load_hdr(sb0, hsc, hd);
   v16f acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -720,13 +749,13 @@ __global__ __launch_bounds__(256, 2) void gemm_s16_kernel(GemmArgs a) {
   v32f zero32;
 #pragma unroll
   for (int r = 0; r < 32; ++r) zero32[r] = 0.0f;
-  fetch(0);
+  fetch(sb0);
   store(0);
   __syncthreads();
 
-  for (int s = 0; s < nsb; ++s) {
-    const int cur = s & 1;
-    const int sn = s + 1 < nsb ? s + 1 : s;
+  for (int s = sb0; s < sb1; ++s) {
+    const int cur = (s - sb0) & 1;
+    const int sn = s + 1 < sb1 ? s + 1 : s;
     fetch(sn);
     const uint32_t scw[4] = {hsc.x, hsc.y, hsc.z, hsc.w};
     const float d = (TYPE == T_Q6_K || TYPE == T_Q3_K || TYPE == T_Q2_K) ? h2f(hd) : h2f(hd) * kIqDScale<TYPE>;
@@ -828,6 +857,10 @@ __global__ __launch_bounds__(256, 2) void gemm_s16_kernel(GemmArgs a) {
   }
   if constexpr (DUMP) return;
   const bool col_ok = n_loc < n_rows;
+  if (CUT && piece >= 0) {
+    store_piece<MT>(a, piece, wave, hf, lc, acc);
+    return;
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -986,15 +1019,56 @@ static hipError_t go_down_rw(const GemmArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// C (op)= the pieces' sums, four columns a thread
+__global__ __launch_bounds__(256) void split_sum_kernel(GemmArgs a, int bm, int gx, int gy, int m_fast) {
+  const int per = bm * 128 / 1024, tile = a.split_from + (int)blockIdx.x / per;
+  const int e = ((int)blockIdx.x % per) * 1024 + 4 * (int)threadIdx.x;
+  const int m = bm * (m_fast ? tile % gy : tile / gx) + e / 128, n = 128 * (m_fast ? tile / gy : tile % gx) + e % 128;
+  if (m >= a.M || n >= a.w.rows) return;
+  const float* p = a.part + (size_t)(tile - a.split_from) * a.splits * bm * 128 + e;
+  v4f v = *(const v4f*)p;
+  for (int k = 1; k < a.splits; ++k) v += *(const v4f*)(p + (size_t)k * bm * 128);
+  float* cp = a.C + (size_t)m * a.ldc + a.c_off + n;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (n + i >= a.w.rows) break;
+    if (a.accumulate == 1) {
+      v[i] += cp[i];
+    } else if (a.accumulate == 2) {
+      const float g = cp[i];
+      v[i] *= g / (1.0f + expf(-g));
+    }
+    cp[i] = v[i];
+  }
+}
+
+hipError_t launch_split_sum(const GemmArgs& a, int bm, int tiles, int gx, int gy, bool m_fast, hipStream_t s) {
+  split_sum_kernel<<<dim3((unsigned)((tiles - a.split_from) * (bm * 128 / 1024))), dim3(256), 0, s>>>(a, bm, gx, gy, m_fast);
+  return hipGetLastError();
+}
+
+// grid of a dense launch with cut tiles: the whole tiles, then the pieces of the others
+static unsigned cut_grid(const GemmArgs& a, int tiles) { return (unsigned)(a.split_from + (tiles - a.split_from) * a.splits); }
+
 template <int TYPE, int MT, int MODE, bool DUMP>
 static hipError_t go_s16(const GemmArgs& a, hipStream_t s) {
   const int n_rows = MODE == GEMM_DENSE ? a.w.rows : a.expert_rows;
   const unsigned gx = (unsigned)((n_rows + 127) / 128);
-  const unsigned gy = MODE == GEMM_DENSE      ? (unsigned)((a.M + 32 * MT - 1) / (32 * MT))
-                     : 32 * MT > kMoeTileRows ? (unsigned)((a.max_tiles + 1) / 2)
-                                              : (unsigned)(a.max_tiles * (kMoeTileRows / (32 * MT)));
-  gemm_s16_kernel<TYPE, MT, MODE, DUMP><<<dim3(gx, gy), dim3(256), 0, s>>>(a);
-  return hipGetLastError();
+  if constexpr (MODE == GEMM_DENSE) {
+    const int gy = (a.M + 32 * MT - 1) / (32 * MT), tiles = (int)gx * gy;
+    if constexpr (!DUMP)
+      if (a.part) {
+        gemm_s16_kernel<TYPE, MT, MODE, DUMP, true><<<dim3(cut_grid(a, tiles)), dim3(256), 0, s>>>(a);
+        return launch_split_sum(a, 32 * MT, tiles, (int)gx, gy, true, s);
+      }
+    gemm_s16_kernel<TYPE, MT, MODE, DUMP><<<dim3((unsigned)tiles), dim3(256), 0, s>>>(a);
+    return hipGetLastError();
+  } else {
+    const unsigned gy = 32 * MT > kMoeTileRows ? (unsigned)((a.max_tiles + 1) / 2)
+                                               : (unsigned)(a.max_tiles * (kMoeTileRows / (32 * MT)));
+    gemm_s16_kernel<TYPE, MT, MODE, DUMP><<<dim3(gx, gy), dim3(256), 0, s>>>(a);
+    return hipGetLastError();
+  }
 }
 
 // zeroes C[m][c_off .. c_off + n) for m < M (a kernel, not a memset, so the call stays capturable in a HIP graph)
@@ -1007,20 +1081,30 @@ template <int TYPE, int MT, int MODE, bool DUMP>
 static hipError_t go(const GemmArgs& a, hipStream_t s) {
   const int n_rows = MODE == GEMM_DENSE ? a.w.rows : a.expert_rows;
   const unsigned gx = (unsigned)((n_rows + 127) / 128);
-  const unsigned gy = MODE == GEMM_DENSE      ? (unsigned)((a.M + 32 * MT - 1) / (32 * MT))
-                     : 32 * MT > kMoeTileRows ? (unsigned)((a.max_tiles + 1) / 2)
-                                              : (unsigned)(a.max_tiles * (kMoeTileRows / (32 * MT)));
-  // A dense product with too few tiles to give every CU two work-groups (M = 512, N = 5120: 320 tiles) splits K in two:
-  // each half adds its partial sums into a zeroed C, so the grid doubles. Two partials keep the result deterministic
-  // (0 + x + y rounds the same in either order); only with accumulate = 0 (C + x + y would not).
-  unsigned gz = 1;
-  if (MODE == GEMM_DENSE && !DUMP && a.accumulate == 0 && gx * gy < 512 && a.w.K / 256 >= 8) {
-    gz = 2;
-    zero_rows_kernel<<<dim3((unsigned)((n_rows + 255) / 256), (unsigned)a.M), dim3(256), 0, s>>>(a.C, a.ldc, a.c_off,
-                                                                                                   n_rows, a.M);
+  if constexpr (MODE == GEMM_DENSE) {
+    const int gy = (a.M + 32 * MT - 1) / (32 * MT), tiles = (int)gx * gy;
+    if constexpr (!DUMP)
+      if (a.part) {
+        gemm_kernel<TYPE, MT, MODE, DUMP, true><<<dim3(cut_grid(a, tiles)), dim3(256), 0, s>>>(a);
+        return launch_split_sum(a, 32 * MT, tiles, (int)gx, gy, true, s);
+      }
+    // Where no tile is cut, a product with too few tiles to give every CU two work-groups splits K in two:
+    // each half adds its partial sums into a zeroed C, so the grid doubles. Two partials keep the result deterministic
+    // (0 + x + y rounds the same in either order); only with accumulate = 0 (C + x + y would not).
+    unsigned gz = 1;
+    if (!DUMP && a.accumulate == 0 && tiles < kGemmSlots && a.w.K / 256 >= 8) {
+      gz = 2;
+      zero_rows_kernel<<<dim3((unsigned)((n_rows + 255) / 256), (unsigned)a.M), dim3(256), 0, s>>>(a.C, a.ldc, a.c_off,
+                                                                                                     n_rows, a.M);
+    }
+    gemm_kernel<TYPE, MT, MODE, DUMP><<<dim3((unsigned)tiles, 1, gz), dim3(256), 0, s>>>(a);
+    return hipGetLastError();
+  } else {
+    const unsigned gy = 32 * MT > kMoeTileRows ? (unsigned)((a.max_tiles + 1) / 2)
+                                               : (unsigned)(a.max_tiles * (kMoeTileRows / (32 * MT)));
+    gemm_kernel<TYPE, MT, MODE, DUMP><<<dim3(gx, gy, 1), dim3(256), 0, s>>>(a);
+    return hipGetLastError();
   }
-  gemm_kernel<TYPE, MT, MODE, DUMP><<<dim3(gx, gy, gz), dim3(256), 0, s>>>(a);
-  return hipGetLastError();
 }
 
 template <int TYPE>
@@ -1069,6 +1153,17 @@ static hipError_t dispatch_s16(int mode, const GemmArgs& a, hipStream_t s) {
     case GEMM_MOE_DOWN: return go_s16<TYPE, 2, GEMM_MOE_DOWN, false>(a, s);
     default: return hipErrorInvalidValue;  // (gate and up in one launch: the int8 kernel's GATEUP mode only)
   }
+}
+
+GemmSplit gemm_split_for(int type, int M, int rows, int K) {
+  if (skinny_supported(type, true, M, rows, K)) return GemmSplit{0, 1, 0};
+  const int gx = (rows + 127) / 128, bm = f16_gemm_supported(type, M, K) ? 128 : M <= 32 ? 32 : 64;
+  const bool s16 = type == T_Q6_K || type == T_Q3_K || type == T_Q2_K || type == T_IQ1_M || type == T_IQ2_XS || type == T_IQ2_S;
+  // (a work-group alone on its CU: the int8 kernel's round takes half of a full one's time, the other two kernels' three quarters:
+  //  IQ4_XS 777 x 17408 -> 5120 357 us of 250 + 107, Q6_K 333 x 17408 -> 5120 301 of 400, Q4_K 512 x 5120 -> 5120 85 of 118)
+  const bool int8 = bm != 128 && !s16;
+  // (a call that takes a workspace costs the host about 28 us, 20 of them the pool's; the f16 path has one anyway)
+  return gemm_split(gx * ((M + bm - 1) / bm), K / 256, bm, int8, int8 ? 0.5f : 0.75f, int8 ? 3.9f : 5.9f, bm == 128 ? 0.0f : 28.0f);
 }
 
 hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s) {

@@ -115,6 +115,8 @@ struct F16Args {
   int ash;             // asc row of 32-block b: b >> ash (per-32 scales: 0; per-256: 3)
   float* C;
   int ldc, c_off, accumulate;
+  float* part;         // partial tiles of the cut tiles (tiles from split_from on, in `splits` pieces of K), or null
+  int split_from, splits;
   int32_t* dbg_isum;   // non-null: write the exact block sums sc * isum [M][rows][K/32] instead of C
 };
 
@@ -151,21 +153,30 @@ __device__ __forceinline__ void q4k_f16_decode(uint32_t x, uint32_t y, int sc, u
   }
 }
 
-// Work-group -> (128-row weight tile, 128-token tile); consecutive work-groups of one XCD (work-groups are dealt to
+// Work-group -> (128-row weight tile, 128-token tile, K piece); consecutive work-groups of one XCD (work-groups are dealt to
 // the 8 XCDs round-robin) take neighbouring weight tiles of one token tile, so the token tile stays in that XCD's L2.
-__device__ __forceinline__ void f16_tile(int& nt, int& mt) {
-  const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
-  int lin = blockIdx.y * gx + blockIdx.x;
-  if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
+// Returns the index of the piece among the cut tiles' pieces, or -1 for a whole tile.
+template <bool CUT>
+__device__ __forceinline__ int f16_tile(const F16Args& a, int& nt, int& mt) {
+  const int gx = (a.w.rows + kF16BN - 1) / kF16BN;
+  int lin = blockIdx.x, piece = -1;
+  const int whole = CUT ? a.split_from : (int)gridDim.x;
+  if (CUT && lin >= whole) {
+    piece = lin - whole;
+    lin = whole + piece / a.splits;
+  } else if (whole % 8 == 0) {
+    lin = (lin % 8) * (whole / 8) + lin / 8;
+  }
   mt = lin / gx;
   nt = lin % gx;
+  return piece;
 }
 
 // S256: per-256 activation scales (the reference's act32 = false, gemm.cl:413-447): one scale per token and superblock,
 // so the f16 MFMAs accumulate the whole superblock's products (sum_b sc * isum, in f32: exact while the partial sums
 // stay below 2^24, i.e. for all but extreme rows, and within f32 rounding otherwise) and the scale is applied once per
 // superblock, res = fma(d * asc, I, fma(-dmin, tmn, res)) -- no per-block VALU work.
-template <int TYPE, bool DUMP, bool S256 = false>
+template <int TYPE, bool DUMP, bool S256 = false, bool CUT = false>
 __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
   // two activation stages of 16 KB, reused at the end to transpose the result tiles (4 waves x 32 x 33 floats)
   __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kF16PairBytes];
@@ -174,7 +185,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, lc = lane & 31;
   const int K = a.w.K, nb = K / 32, nsb = K / 256, npair = K / 64;
   int nt, mt;
-  f16_tile(nt, mt);
+  const int piece = f16_tile<CUT>(a, nt, mt);
+  const int z = CUT && piece >= 0 ? piece % a.splits : 0, nz = CUT && piece >= 0 ? a.splits : 1;
+  const int sb0 = z * nsb / nz, sb1 = (z + 1) * nsb / nz;  // (its piece of a cut tile, or all superblocks)
   const int m0 = mt * kF16BM;
   const int n_rows = a.w.rows;
   const int nbase = nt * kF16BN + wave * 32;
@@ -213,23 +226,23 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
     for (int r = 0; r < 16; ++r) res[t][r] = 0.0f;
   const f32x16 zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
-  uint4 hdr = *(const uint4*)hrow, hdr_n;
+  uint4 hdr = *(const uint4*)(hrow + (size_t)sb0 * 16), hdr_n;
   uint2 pay[2], pay_n[2];
 #pragma unroll
-  for (int bb = 0; bb < 2; ++bb) pay[bb] = *(const uint2*)(qrow + bb * 16);
-  fetch_sa(0);
-  fetch(0);
+  for (int bb = 0; bb < 2; ++bb) pay[bb] = *(const uint2*)(qrow + (size_t)(8 * sb0 + bb) * 16);
+  fetch_sa(4 * sb0);
+  fetch(4 * sb0);
   store(0);
   store_sa(0);
   __syncthreads();
 
-  for (int s = 0; s < nsb; ++s) {
-    const int sn = s + 1 < nsb ? s + 1 : s;
+  for (int s = sb0; s < sb1; ++s) {
+    const int sn = s + 1 < sb1 ? s + 1 : s;
     hdr_n = *(const uint4*)(hrow + (size_t)sn * 16);
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const int g = 4 * s + p, cur = g & 1;
-      const int gn = g + 1 < npair ? g + 1 : g;
+      const int gn = g + 1 < 4 * sb1 ? g + 1 : g;
       fetch(gn);
 #pragma unroll
       for (int bb = 0; bb < 2; ++bb) pay_n[bb] = *(const uint2*)(qrow + (size_t)(2 * gn + bb) * 16);
@@ -393,6 +406,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
     for (int k = 0; k < 16; ++k) {
       const int ml = 2 * k + h, m = m0 + 32 * t + ml;
       const float v0 = T[lc * 33 + ml];
+      if (CUT && piece >= 0) {  // (piece-local [128 tokens][128 rows])
+        a.part[(size_t)piece * (kF16BM * kF16BN) + (32 * t + ml) * kF16BN + wave * 32 + lc] = v0;
+        continue;
+      }
       if (m < a.M && n < n_rows) {
         float* cp = a.C + (size_t)m * a.ldc + a.c_off + n;
         float v = v0;
@@ -418,7 +435,7 @@ bool f16_gemm_supported(int type, int M, int K) {
 
 // One memory pool per device for the per-call workspace (stream-ordered: concurrent calls on different streams get
 // different buffers; the pool keeps freed memory for the next call).
-static hipError_t f16_pool(hipMemPool_t* out) {
+static hipError_t call_pool(hipMemPool_t* out) {
   static std::mutex mu;
   static hipMemPool_t pools[64] = {};
   int dev = 0;
@@ -443,29 +460,39 @@ static hipError_t f16_pool(hipMemPool_t* out) {
   return hipSuccess;
 }
 
+hipError_t pool_alloc(void** out, size_t bytes, hipStream_t s) {
+  hipMemPool_t pool = nullptr;
+  const hipError_t e = call_pool(&pool);
+  return e == hipSuccess ? hipMallocFromPoolAsync(out, bytes, pool, s) : e;
+}
+
 // Allocation-free workspace for qmatmul_gemm_noalloc: a file-scope device array (each GPU holds its own copy until
 // the process ends). Host code never passes the array's name to a kernel or a copy -- in host code it is only a
 // stand-in for the symbol -- but the device address that hipGetSymbolAddress returns for the current device, looked
 // up once per device (under a lock) and kept.
 constexpr size_t kF16ScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) uint8_t scratch[kF16ScratchBytes];
+static __device__ __align__(256) uint8_t split_scratch[kSplitBytes];  // (partial tiles of the cut tiles)
 
-hipError_t f16_scratch(void** out, size_t* bytes) {
+hipError_t f16_scratch(void** out, size_t* bytes, void** part) {
   static std::mutex mu;
-  static void* ptrs[64] = {};
+  static void *ptrs[64] = {}, *parts[64] = {};
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
   std::lock_guard<std::mutex> lock(mu);
   if (!ptrs[dev]) {
-    void* p = nullptr;
+    void *p = nullptr, *q = nullptr;
     e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+    if (e == hipSuccess) e = hipGetSymbolAddress(&q, HIP_SYMBOL(split_scratch));
     if (e != hipSuccess) return e;
     ptrs[dev] = p;
+    parts[dev] = q;
   }
   *out = ptrs[dev];
   *bytes = kF16ScratchBytes;
+  *part = parts[dev];
   return hipSuccess;
 }
 
@@ -476,9 +503,7 @@ hipError_t launch_gemm_f16(int type, const GemmArgs& g, void* ws, hipStream_t s)
   void* buf = ws;
   hipError_t e = hipSuccess;
   if (!buf) {
-    hipMemPool_t pool = nullptr;
-    e = f16_pool(&pool);
-    if (e == hipSuccess) e = hipMallocFromPoolAsync(&buf, f16_workspace_bytes(M, K), pool, s);
+    e = pool_alloc(&buf, f16_workspace_bytes(M, K), s);
     if (e != hipSuccess) return e;
   }
   uint8_t* af = (uint8_t*)buf;
@@ -506,11 +531,18 @@ hipError_t launch_gemm_f16(int type, const GemmArgs& g, void* ws, hipStream_t s)
     a.c_off = g.c_off;
     a.accumulate = g.accumulate;
     a.dbg_isum = g.dbg_isum;
-    const dim3 grid((unsigned)((g.w.rows + kF16BN - 1) / kF16BN), (unsigned)(Mp / kF16BM));
+    a.part = g.part;
+    a.split_from = g.split_from;
+    a.splits = g.splits;
+    const int gx = (g.w.rows + kF16BN - 1) / kF16BN, gy = Mp / kF16BM, tiles = gx * gy;
+    const dim3 grid((unsigned)(g.part ? g.split_from + (tiles - g.split_from) * g.splits : tiles));
     if (g.dbg_isum) gemm_f16_kernel<T_Q4_K, true><<<grid, dim3(256), 0, s>>>(a);
+    else if (g.ash == 3 && g.part) gemm_f16_kernel<T_Q4_K, false, true, true><<<grid, dim3(256), 0, s>>>(a);
     else if (g.ash == 3) gemm_f16_kernel<T_Q4_K, false, true><<<grid, dim3(256), 0, s>>>(a);
+    else if (g.part) gemm_f16_kernel<T_Q4_K, false, false, true><<<grid, dim3(256), 0, s>>>(a);
     else gemm_f16_kernel<T_Q4_K, false><<<grid, dim3(256), 0, s>>>(a);
     e = hipGetLastError();
+    if (e == hipSuccess && g.part) e = launch_split_sum(g, kF16BM, tiles, gx, gy, false, s);
   }
   if (!ws) {
     const hipError_t e2 = hipFreeAsync(buf, s);

@@ -2,6 +2,7 @@
 // All return hipSuccess or the launch error; shapes are validated by the C-ABI layer (qm_api.hip) beforehand.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 #include "qm_device.h"
@@ -61,6 +62,10 @@ struct GemmArgs {
   float* C;
   int ldc, c_off, accumulate;
   int32_t* dbg_isum;
+  // Dense products: tiles from split_from on are cut into `splits` pieces of K each, whose partial tiles go to part (see
+  // gemm_split); part null: no tile is cut
+  float* part = nullptr;
+  int split_from = 0, splits = 1;
   int ash = 0;  // activation scales per 32 << ash values: asc row of 32-block b is b >> ash (0, or 3 = per 256)
   // MoE tile mode
   const int* tiles;    // [0] = count, then (expert, first slot, rows) per tile
@@ -74,6 +79,57 @@ struct GemmArgs {
 };
 // MoE tile modes: GATEUP (gate and up of one type in one launch: h quantized), G (gate alone: f32 g into C),
 // UH (up alone after G: h from u and g, quantized), DOWN (routing-weighted y)
+// How a dense product's tiles are dealt. The chip holds kGemmSlots work-groups of the prompt kernels at once (two per CU), so
+// tiles run in rounds and the last one is often nearly empty (520 tiles take the time of 1024). The tiles past the last
+// whole round -- all of them for a small product -- are cut along K into `splits` pieces, each with its share of the
+// superblocks, whose partial tiles are added by a second kernel (in piece order: the result does not depend on timing).
+constexpr int kGemmSlots = 512;
+constexpr size_t kSplitBytes = (size_t)32 << 20;  // most partial tiles of one call
+struct GemmSplit {
+  int from, splits;  // tiles [0, from) whole, [from, tiles) in `splits` pieces each (splits = 1: none)
+  size_t bytes;      // partial tiles
+};
+// Rounds that n equal work-groups take; alone: the time of a round that fills half the slots or less (a work-group that has
+// its CU to itself runs faster than two that share it), as a part of a full one
+inline float gemm_rounds(int n, float alone) {
+  const int rem = n % kGemmSlots;
+  return (float)(n / kGemmSlots) + (rem == 0 ? 0.0f : 2 * rem <= kGemmSlots ? alone : 1.0f);
+}
+// tiles of bm x 128 results, K of nsb superblocks; us: microseconds of a full round's superblock; host: those below which the
+// call would wait for its own workspace (0: it has one anyway); halves: uncut, a small product's two K halves are added into a zeroed C.
+// With more than one whole round the last one starts while others still run, and cutting it measured level (Q4_K 2048 x 5120 ->
+// 17408, 2176 tiles: 572 us either way), so only products of fewer than 1024 tiles are cut.
+inline GemmSplit gemm_split(int tiles, int nsb, int bm, bool halves, float alone, float us, float host) {
+  GemmSplit r{tiles, 1, 0};
+  const int full = tiles / kGemmSlots * kGemmSlots, rem = tiles - full;
+  if (rem == 0 || full > kGemmSlots) return r;
+  // time of the tail in superblocks per slot: a piece costs its superblocks and about one more (its prologue and store), the
+  // second kernel about 1.5 and the partial tiles' traffic 1.4 per 512 pieces of 64 x 128 results. Cut for a tenth or more.
+  float best = gemm_rounds(rem, alone) * (float)nsb;
+  if (halves && tiles < kGemmSlots && nsb >= 8) best = fminf(best, gemm_rounds(2 * rem, alone) * (float)(nsb / 2 + 1) + 2.0f);
+  const float uncut = (best + (float)(full / kGemmSlots * nsb)) * us;
+  best = 0.9f * best;
+  for (int s = 2; s <= 8 && nsb / s >= 2; ++s) {
+    const size_t bytes = (size_t)rem * s * bm * 128 * sizeof(float);
+    const float t = gemm_rounds(rem * s, alone) * ((float)((nsb + s - 1) / s) + 1.0f) + 1.5f +
+                    1.4f * (float)(rem * s) * (float)bm / (64.0f * 512.0f);
+    const float cut = (t + (float)(full / kGemmSlots * nsb)) * us;
+    if (host > 0.0f && uncut - fmaxf(cut, host) < 8.0f) continue;
+    if (t < best && bytes <= kSplitBytes) {
+      best = t;
+      r = GemmSplit{full, s, bytes};
+    }
+  }
+  return r;
+}
+// The same for one call: the kernel that launch_gemm / launch_gemm_f16 takes for it (splits = 1 where it takes another)
+GemmSplit gemm_split_for(int type, int M, int rows, int K);
+// C (op)= the sums of the cut tiles' pieces (bm x 128 each); tile t: rows bm * (t % gy).., columns 128 * (t / gy).. when
+// m_fast, else bm * (t / gx).., 128 * (t % gx)..
+hipError_t launch_split_sum(const GemmArgs& a, int bm, int tiles, int gx, int gy, bool m_fast, hipStream_t s);
+// A per-device stream-ordered memory pool for per-call workspaces
+hipError_t pool_alloc(void** out, size_t bytes, hipStream_t s);
+
 enum GemmMode : int { GEMM_DENSE = 0, GEMM_MOE_GATEUP = 1, GEMM_MOE_DOWN = 2, GEMM_MOE_G = 3, GEMM_MOE_UH = 4 };
 hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s);
 // Prompt GEMM on the f16 matrix pipe (qm_gemm_f16.hip): the types and shapes it takes, its per-call workspace, and
@@ -81,8 +137,9 @@ hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s);
 bool f16_gemm_supported(int type, int M, int K);
 size_t f16_workspace_bytes(int M, int K);
 hipError_t launch_gemm_f16(int type, const GemmArgs& a, void* ws, hipStream_t s);
-// The current device's copy of the static scratch array (device address and size) for the allocation-free entry
-hipError_t f16_scratch(void** ptr, size_t* bytes);
+// The current device's copies of the static scratch arrays for the allocation-free entry: ptr (bytes) the f16 path's
+// workspace, part (kSplitBytes) the partial tiles
+hipError_t f16_scratch(void** ptr, size_t* bytes, void** part);
 // slots per MoE tile (one expert each); a 64-row tile (fewer, larger tiles) measured slower under the Zipf skew
 constexpr int kMoeTileRows = 32;
 

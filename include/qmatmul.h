@@ -146,7 +146,9 @@ int qmatmul_gemv(const qm_weight* w, const int8_t* aq, const float* asc, const i
  * gemm_ext (zero/engine.h:3234-3297; zero/kernels/gemm.cl:132-475). Q4_K is computed exactly (scales and mins),
  * not requantized as the reference's W8 path does (zero/kernels/decode.cl:455-507). Q4_K with M >= 128 runs on the
  * f16 matrix pipe (exact integer block sums from f16 products) and takes a per-call workspace of about 2*M*K bytes
- * from a per-device stream-ordered memory pool; every other case runs on int8 MFMA and allocates nothing. A caller
+ * from a per-device stream-ordered memory pool; every other case runs on int8 MFMA. Products of few tiles, or of few more
+ * than the chip holds at once, are cut along K and take up to 32 MiB of that pool for the pieces' partial results (not on a
+ * stream under capture, nor when the pool has none: they then run uncut, equal up to f32 rounding order). A caller
  * that owns all memory passes the workspace itself (qmatmul_gemm_ws). */
 int qmatmul_gemm(const qm_weight* w, const int8_t* aq, const float* asc, const int16_t* absum, int M, int M_stride,
                  float* C, int ldc, int c_off, int accumulate, void* stream);
@@ -159,20 +161,22 @@ int qmatmul_gemm_ex(const qm_weight* w, const int8_t* aq, const float* asc, cons
                     int act32, float* C, int ldc, int c_off, int accumulate, void* stream);
 
 /* The prompt GEMM with a caller-owned workspace, as the reference's engine owns its W8 staging buffers
- * (zero/engine.h:3238-3246): qmatmul_gemm_ex's arguments plus ws (device, 256-byte aligned) of at least
- * qmatmul_gemm_workspace_size(w, M) bytes. That size is 0 for every call but Q4_K with M >= 128 (then
- * 2*Mp*K + 4*Mp*K/32 bytes, Mp = M rounded up to 128); ws may be NULL when it is 0. No allocation, no host
- * synchronisation; calls on different streams need different workspaces. QM_ERR_WORKSPACE if ws is too small. */
+ * (zero/engine.h:3238-3246): qmatmul_gemm_ex's arguments plus ws (device, 256-byte aligned) of
+ * qmatmul_gemm_workspace_size(w, M) bytes: what qmatmul_gemm takes from its pool, 0 for many calls (ws may then be NULL).
+ * Only Q4_K with M >= 128 must have one, of at least 2*Mp*K + 4*Mp*K/32 bytes (Mp = M rounded up to 128;
+ * QM_ERR_WORKSPACE if ws is smaller); the rest of the size is for partial results, without which a call runs uncut. No
+ * allocation, no host synchronisation; calls on different streams need different workspaces. */
 size_t qmatmul_gemm_workspace_size(const qm_weight* w, int M);
 int qmatmul_gemm_ws(const qm_weight* w, const int8_t* aq, const float* asc, const int16_t* absum, int M, int M_stride,
                     int act32, float* C, int ldc, int c_off, int accumulate, void* ws, size_t ws_bytes, void* stream);
 
 /* qmatmul_gemm without any device allocation. No counterpart in the reference: for callers that cannot allocate
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc). Same arguments, results and kernels
- * as qmatmul_gemm; where qmatmul_gemm would take its pool workspace, this entry uses a static 32 MiB device array
- * (one per GPU, held until the process ends) and returns QM_ERR_WORKSPACE when the call needs more
- * (f16 path: 2*Mp*K + 4*Mp*K/32 bytes, Mp = M rounded up to 128; e.g. M 2048 x K 5120 needs 22.3 MB).
- * Every call on one GPU shares that GPU's array: calls that overlap on one GPU (different streams, or threads) race
+ * as qmatmul_gemm; where qmatmul_gemm would take its pool workspace, this entry uses two static 32 MiB device arrays
+ * (on each GPU, held until the process ends), one for the f16 path, one for partial results, and returns
+ * QM_ERR_WORKSPACE when the f16 path needs more
+ * (2*Mp*K + 4*Mp*K/32 bytes, Mp = M rounded up to 128; e.g. M 2048 x K 5120 needs 22.3 MB).
+ * Every call on one GPU shares that GPU's arrays: calls that overlap on one GPU (different streams, or threads) race
  * and must be ordered by the caller. Each call writes every scratch byte it reads before reading it. It takes per-32
  * activation scales only (qmatmul_gemm's act32 = 1); a caller with per-256 scales that cannot allocate passes its
  * own workspace to qmatmul_gemm_ws. */

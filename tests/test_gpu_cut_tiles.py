@@ -1,0 +1,78 @@
+"""Prompt products whose tiles are cut along K into pieces (partial tiles added by a second kernel): against the CPU oracle at
+ragged tile edges, every accumulate mode, and the three entry points bit for bit the same where all have the room."""
+import numpy as np
+import pytest
+
+import oracle
+from arcinfer_amd import formats as F
+
+from .test_gpu_parity import TOL_INT8_PATH, acts, assert_elementwise, rel_err, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# (type, M, N, K): the f16, int8 and per-16 kernels; partial row and column tiles; superblocks that do not divide evenly over
+# the pieces; 522 tiles, of which the last ten are cut
+CASES = [(F.Q4_K, 130, 144, 2048), (F.Q4_K, 300, 272, 5888), (F.IQ4_XS, 70, 272, 8192), (F.IQ3_S, 64, 144, 17408),
+         (F.Q6_K, 70, 272, 2304), (F.Q2_K, 129, 144, 4096), (F.IQ4_XS, 520, 7376, 4096), (F.Q6_K, 520, 7376, 2816)]
+
+
+@pytest.mark.parametrize("qtype,M,N,K", CASES)
+def test_cut_tiles(qm, dev, qtype, M, N, K):
+    import torch
+    W = F.synth_weight(qtype, N, K, seed=qtype + M)
+    aq, asc, absum = acts(qm, F.synth_activations(M, K, seed=K, outlier_frac=0.01), dev, M_stride=M + 3)
+    w = qm.QWeight(qtype, to_dev(W, dev), N, K)
+    need = qm.gemm_workspace_size(w, M)
+    assert need > (2 * M * K if qtype == F.Q4_K else 0)  # (room for partial tiles: the call is cut)
+    C = qm.gemm(w, aq, asc, absum, M=M)
+    ws = torch.empty((need,), dtype=torch.uint8, device=dev)
+    assert torch.equal(C, qm.gemm_ws(w, aq, asc, absum, ws, M=M))
+    assert torch.equal(C, qm.gemm(w, aq, asc, absum, M=M, noalloc=True))
+    g = torch.randn((M, N + 8), device=dev)
+    add = qm.gemm(w, aq, asc, absum, M=M, C=g.clone(), ldc=N + 8, c_off=5, accumulate=1)
+    mul = qm.gemm(w, aq, asc, absum, M=M, C=g.clone(), ldc=N + 8, c_off=5, accumulate=2)
+    torch.cuda.synchronize()
+    stride = max(1, N // 256)
+    ref = oracle.blockdot(qtype, W, K, aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy(), M=M, col_stride=stride)
+    sel = np.arange(0, N, stride)
+    got = C.cpu().numpy()[:, sel]
+    ref = ref[:, sel] if ref.shape[1] == N else ref
+    assert rel_err(got, ref) < TOL_INT8_PATH
+    assert_elementwise(got, ref)
+    assert torch.equal(add[:, 5:5 + N], g[:, 5:5 + N] + C)
+    assert torch.allclose(mul[:, 5:5 + N], torch.nn.functional.silu(g[:, 5:5 + N]) * C, rtol=1e-5,
+                          atol=1e-6 * C.abs().max().item())
+    for t in (add, mul):
+        assert torch.equal(t[:, :5], g[:, :5]) and torch.equal(t[:, 5 + N:], g[:, 5 + N:])
+
+
+@pytest.mark.parametrize("qtype", [F.IQ4_XS, F.Q6_K])
+def test_no_workspace_is_accepted(qm, dev, qtype):
+    """The kernels that need no workspace run without one (uncut: equal up to the f32 order of the K pieces)."""
+    import torch
+    M, N, K = 70, 272, 8192
+    w = qm.QWeight(qtype, to_dev(F.synth_weight(qtype, N, K, seed=1), dev), N, K)
+    aq, asc, absum = acts(qm, F.synth_activations(M, K, seed=2), dev, M_stride=M)
+    C = qm.gemm(w, aq, asc, absum, M=M)
+    D = qm.gemm_ws(w, aq, asc, absum, None, M=M)
+    torch.cuda.synchronize()
+    assert rel_err(D.cpu().numpy(), C.cpu().numpy()) < 1e-5
+
+
+def test_captured_call_matches(qm, dev):
+    """Under stream capture the int8 kernels record no allocation; every replay gives the eager uncut result."""
+    import torch
+    M, N, K = 70, 272, 8192
+    w = qm.QWeight(F.IQ4_XS, to_dev(F.synth_weight(F.IQ4_XS, N, K, seed=1), dev), N, K)
+    aq, asc, absum = acts(qm, F.synth_activations(M, K, seed=2), dev, M_stride=M)
+    want = qm.gemm_ws(w, aq, asc, absum, None, M=M)
+    C = torch.empty((M, N), device=dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        qm.gemm(w, aq, asc, absum, M=M, C=C)
+    for _ in range(3):
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
