@@ -642,7 +642,8 @@ int qmatmul_moe_grouped_ex(const qm_weight* gate, const qm_weight* up, const qm_
   // gate and up: one launch when they share a type the int8 kernel takes in one pass; otherwise the gate projection
   // into hf, then the up projection forming h from it
   const bool s16 = [](int t) { return t == QM_Q6_K || t == QM_IQ2_XS || t == QM_IQ2_S || t == QM_Q3_K; }(gate->type);
-  const bool fused = gate->type == up->type && !s16;
+  const bool few = gate->type == up->type && qm::moe_few(gate->type, L.slots, NE, Fv);
+  const bool fused = gate->type == up->type && (!s16 || few);
   if (e == hipSuccess) {
     qm::GemmArgs a{};
     a.w = gate->view;
@@ -660,7 +661,9 @@ int qmatmul_moe_grouped_ex(const qm_weight* gate, const qm_weight* up, const qm_
     a.expert_rows = Fv;
     a.C = hf;
     a.ldc = F;
-    if (fused) {
+    if (few) {
+      e = qm::launch_moe_few(gate->type, false, a, s);
+    } else if (fused) {
       e = qm::launch_gemm(gate->type, qm::GEMM_MOE_GATEUP, a, s);
     } else {
       e = qm::launch_gemm(gate->type, qm::GEMM_MOE_G, a, s);
@@ -685,7 +688,7 @@ int qmatmul_moe_grouped_ex(const qm_weight* gate, const qm_weight* up, const qm_
     a.slots = L.slots;
     a.max_tiles = L.max_tiles;
     a.expert_rows = E;
-    e = qm::launch_gemm(down->type, qm::GEMM_MOE_DOWN, a, s);
+    e = few ? qm::launch_moe_few(down->type, true, a, s) : qm::launch_gemm(down->type, qm::GEMM_MOE_DOWN, a, s);
   }
   if (e == hipSuccess) e = qm::launch_moe_combine(x, y, inv, T, NU, E, accumulate, shd, s);
   return e == hipSuccess ? QM_OK : hip_fail(e, "qmatmul_moe_grouped");

@@ -177,6 +177,10 @@ hipError_t launch_moe_scan(int* part, int groups, int* counts, int NE, hipStream
 hipError_t launch_moe_scatter(const int* ids, const float* wts, int T, int NU, int NE, const int* part,
                               const int* counts, int* cursor, int* tstart, int* tiles, int tile_rows, int* stok,
                               float* swt, int* inv, hipStream_t s);
+// Expert products over the slot tiles for small expert sets (qm_moe_few.hip): gate and up of one type (hq / hsc), or down; and
+// whether a layer of `slots` slots, NE experts and expert width Fv takes them
+bool moe_few(int type, int slots, int NE, int Fv);
+hipError_t launch_moe_few(int type, bool down, const GemmArgs& a, hipStream_t s);
 hipError_t launch_moe_combine(float* x, const float* y, const int* inv, int T, int NU, int E, int accumulate,
                               const MoeShared& sh, hipStream_t s);
 hipError_t launch_fill_i32(int* p, int value, size_t n, hipStream_t s);
