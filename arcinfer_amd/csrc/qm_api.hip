@@ -427,43 +427,53 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   a.accumulate = accumulate;
   a.ash = act32 ? 0 : 3;
   hipError_t e;
-  const bool f16 = qm::f16_gemm_supported(w->type, M, w->view.K);
-  const size_t need = f16 ? align256(qm::f16_workspace_bytes(M, w->view.K)) : 0;  // the f16 path's activations
-  const qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, w->view.K);
-  const size_t pb = sp.splits > 1 ? sp.bytes : 0;                                 // partial tiles (optional)
-  void *scr = nullptr, *pool = nullptr;
+  const int K = w->view.K;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const bool capturing = wm == WS_POOL && (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone);
+  void *scr = nullptr, *static_part = nullptr;
+  size_t cap_bytes = 0;
+  if (wm == WS_STATIC) {
+    e = qm::f16_scratch(&scr, &cap_bytes, &static_part);
+    if (e != hipSuccess) return hip_fail(e, "qmatmul_gemm_noalloc: scratch lookup");
+  }
+  // the f16 path's activations: Q4_K must have room for them; the other types of that path run on int8 MFMA without (and on a
+  // capturing stream, where they record no allocation)
+  const size_t fb = qm::f16_workspace_bytes(M, K);
+  bool f16 = qm::f16_gemm_supported(w->type, M, w->rows, K);
+  if (f16 && w->type != QM_Q4_K)
+    f16 = wm == WS_STATIC ? fb <= cap_bytes : wm == WS_CALLER ? ws && ws_bytes >= fb && aligned(ws, 256) : !capturing;
+  if (f16 && wm == WS_STATIC && fb > cap_bytes)
+    return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs %zu bytes of scratch, the static scratch holds %zu "
+                "(use qmatmul_gemm or qmatmul_gemm_ws)", fn, M, K, fb, cap_bytes);
+  if (f16 && wm == WS_CALLER) {
+    if (!ws || ws_bytes < fb)
+      return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs a workspace of %zu bytes (given %zu%s)", fn, M, K, fb, ws_bytes,
+                  ws ? "" : ", null");
+    if (!aligned(ws, 256)) return fail(QM_ERR_ARG, "%s: the workspace must be 256-byte aligned", fn);
+    scr = ws;
+  }
+  size_t need = f16 ? align256(fb) : 0;
+  qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, K, f16);
+  size_t pb = sp.splits > 1 ? sp.bytes : 0;  // partial tiles (optional)
+  void* pool = nullptr;
   float* part = nullptr;
   if (wm == WS_STATIC) {
-    size_t cap = 0;
-    void* ps = nullptr;
-    e = qm::f16_scratch(&scr, &cap, &ps);
-    if (e != hipSuccess) return hip_fail(e, "qmatmul_gemm_noalloc: scratch lookup");
-    if (f16 && qm::f16_workspace_bytes(M, w->view.K) > cap)
-      return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs %zu bytes of scratch, the static scratch holds %zu "
-                  "(use qmatmul_gemm or qmatmul_gemm_ws)", fn, M, w->view.K, need, cap);
-    if (pb) part = (float*)ps;
+    if (pb) part = (float*)static_part;
   } else if (wm == WS_CALLER) {
-    if (f16) {
-      if (!ws || ws_bytes < qm::f16_workspace_bytes(M, w->view.K))
-        return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs a workspace of %zu bytes (given %zu%s)", fn, M,
-                    w->view.K, need, ws_bytes, ws ? "" : ", null");
-      if (!aligned(ws, 256)) return fail(QM_ERR_ARG, "%s: the workspace must be 256-byte aligned", fn);
-      scr = ws;
-    }
     if (pb && ws && ws_bytes >= need + pb && aligned(ws, 256)) part = (float*)((uint8_t*)ws + need);
-  } else if (f16 || pb) {
-    // (a capturing stream: no partial tiles, so the types that need no workspace record no allocation)
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const bool cut = pb && hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
-    if (need || cut) {
-      e = qm::pool_alloc(&pool, need + (cut ? pb : 0), (hipStream_t)stream);
-      if (e != hipSuccess && f16) return hip_fail(e, fn);
+  } else {
+    if (capturing) pb = 0;
+    if (need + pb) {
+      e = qm::pool_alloc(&pool, need + pb, (hipStream_t)stream);
       if (e == hipSuccess) {
-        scr = pool;
-        if (cut) part = (float*)((uint8_t*)pool + need);
+        if (f16) scr = pool;
+        if (pb) part = (float*)((uint8_t*)pool + need);
+      } else if (w->type == QM_Q4_K && f16) {
+        return hip_fail(e, fn);
       } else {
+        (void)hipGetLastError();  // (no memory: the int8 kernels, uncut, need none)
         pool = nullptr;
-        (void)hipGetLastError();  // (no partial tiles then: the uncut kernels need no memory)
+        f16 = false;
       }
     }
   }
@@ -495,8 +505,9 @@ int qmatmul_gemm_ex(const qm_weight* w, const int8_t* aq, const float* asc, cons
 
 size_t qmatmul_gemm_workspace_size(const qm_weight* w, int M) {
   if (!w || M < 1) return 0;
-  const size_t need = qm::f16_gemm_supported(w->type, M, w->view.K) ? qm::f16_workspace_bytes(M, w->view.K) : 0;
-  const qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, w->view.K);
+  const bool f16 = qm::f16_gemm_supported(w->type, M, w->rows, w->view.K);
+  const size_t need = f16 ? qm::f16_workspace_bytes(M, w->view.K) : 0;
+  const qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, w->view.K, f16);
   return sp.splits > 1 ? align256(need) + sp.bytes : need;
 }
 
@@ -525,7 +536,7 @@ int qmatmul_gemm_blocksums(const qm_weight* w, const int8_t* aq, int M, int M_st
   a.M_stride = M_stride;
   a.dbg_isum = isum;
   // (the same kernel choice as qmatmul_gemm makes for this type and shape)
-  const hipError_t e = qm::f16_gemm_supported(w->type, M, w->view.K)
+  const hipError_t e = qm::f16_gemm_supported(w->type, M, w->rows, w->view.K)
                            ? qm::launch_gemm_f16(w->type, a, nullptr, (hipStream_t)stream)
                            : qm::launch_gemm(w->type, qm::GEMM_DENSE, a, (hipStream_t)stream);
   return e == hipSuccess ? QM_OK : hip_fail(e, "qmatmul_gemm_blocksums");

@@ -1088,11 +1088,12 @@ static hipError_t go(const GemmArgs& a, hipStream_t s) {
         gemm_kernel<TYPE, MT, MODE, DUMP, true><<<dim3(cut_grid(a, tiles)), dim3(256), 0, s>>>(a);
         return launch_split_sum(a, 32 * MT, tiles, (int)gx, gy, true, s);
       }
-    // Where no tile is cut, a product with too few tiles to give every CU two work-groups splits K in two:
-    // each half adds its partial sums into a zeroed C, so the grid doubles. Two partials keep the result deterministic
-    // (0 + x + y rounds the same in either order); only with accumulate = 0 (C + x + y would not).
+    // Where no tile is cut, a product with too few tiles to give every CU two work-groups splits K in two (if the doubled grid
+    // then does not take as many rounds: 416 tiles of Q5_K 777 x 4096 -> 4096 93 us in halves): each half adds its partial
+    // sums into a zeroed C. Two partials keep the result deterministic (0 + x + y rounds the same in either order); only with
+    // accumulate = 0 (C + x + y would not).
     unsigned gz = 1;
-    if (!DUMP && a.accumulate == 0 && tiles < kGemmSlots && a.w.K / 256 >= 8) {
+    if (!DUMP && a.accumulate == 0 && gemm_split_for(TYPE, a.M, n_rows, a.w.K, false).halves) {
       gz = 2;
       zero_rows_kernel<<<dim3((unsigned)((n_rows + 255) / 256), (unsigned)a.M), dim3(256), 0, s>>>(a.C, a.ldc, a.c_off,
                                                                                                      n_rows, a.M);
@@ -1155,15 +1156,16 @@ static hipError_t dispatch_s16(int mode, const GemmArgs& a, hipStream_t s) {
   }
 }
 
-GemmSplit gemm_split_for(int type, int M, int rows, int K) {
-  if (skinny_supported(type, true, M, rows, K)) return GemmSplit{0, 1, 0};
-  const int gx = (rows + 127) / 128, bm = f16_gemm_supported(type, M, K) ? 128 : M <= 32 ? 32 : 64;
+// A work-group alone on its CU: the int8 kernel's round takes half of a full one's time, the other two kernels' about 0.7 (IQ4_XS
+// 777 x 17408 -> 5120 357 us of 250 + 107, Q6_K 333 x 17408 -> 5120 301 of 400, Q4_K 1024 x 4096 -> 4096 71 of 101).
+// A call that takes a workspace costs the host about 28 us, 20 of them the pool's; the f16 path has one anyway.
+GemmSplit gemm_split_for(int type, int M, int rows, int K, bool f16) {
+  if (!f16 && skinny_supported(type, true, M, rows, K)) return GemmSplit{0, 1, 0, false, 0.0f};
+  const int gx = (rows + 127) / 128, bm = f16 ? 128 : M <= 32 ? 32 : 64;
   const bool s16 = type == T_Q6_K || type == T_Q3_K || type == T_Q2_K || type == T_IQ1_M || type == T_IQ2_XS || type == T_IQ2_S;
-  // (a work-group alone on its CU: the int8 kernel's round takes half of a full one's time, the other two kernels' three quarters:
-  //  IQ4_XS 777 x 17408 -> 5120 357 us of 250 + 107, Q6_K 333 x 17408 -> 5120 301 of 400, Q4_K 512 x 5120 -> 5120 85 of 118)
-  const bool int8 = bm != 128 && !s16;
-  // (a call that takes a workspace costs the host about 28 us, 20 of them the pool's; the f16 path has one anyway)
-  return gemm_split(gx * ((M + bm - 1) / bm), K / 256, bm, int8, int8 ? 0.5f : 0.75f, int8 ? 3.9f : 5.9f, bm == 128 ? 0.0f : 28.0f);
+  const bool int8 = !f16 && !s16;
+  return gemm_split(gx * ((M + bm - 1) / bm), K / 256, bm, int8, int8 ? 0.5f : f16 ? 0.7f : 0.75f, int8 ? 4.2f : f16 ? 6.5f : 5.9f,
+                    f16 ? 0.0f : 28.0f);
 }
 
 hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s) {

@@ -50,13 +50,19 @@ size_t f16_workspace_bytes(int M, int K) {
   return round_up(Mp * (size_t)K * 2, 256) + Mp * (size_t)(K / 32) * 4;
 }
 
+// The types of this kernel: Q4_K (Q5_K's and IQ3_S's values times their integer block scales fit an f16 exactly too: 31 * 63 =
+// 1953, 15 * 31 = 465). kF16Half: see f16_act_kernel.
+template <int TYPE> constexpr bool kF16Half = TYPE == T_Q5_K || TYPE == T_IQ3_S;
+
 // ---- prepass: the int8 activations as f16 in MFMA operand order, and (MINS) the mins operand u = asc * bsum split
 // into two bf16 parts (one 32-bit word per token and block: bf16 hi | lo << 16; per superblock the 8 words are the
 // bf16 MFMA's B operand, slot 8h + i = block 4h + i / 2, part i % 2).
 // One thread per (token, 32-block, k-half h); consecutive threads take consecutive lanes of one operand piece
 // (token % 32, then h), so each wave writes whole 1 KB pieces. A thread writes lane (token % 32, h)'s 16 bytes of the
 // block's two pieces: chunk c = 0 holds elements 8h + perm8(i), chunk 1 elements 16 + 8h + perm8(i).
-template <bool MINS>
+// HALF: lane half h holds the 16 elements of half h (chunk c: 16h + 8c + perm8(i)) instead, for the types whose records keep
+// a half together (kF16Half).
+template <bool MINS, bool HALF>
 __global__ __launch_bounds__(256) void f16_act_kernel(const int8_t* aq, const float* asc, const int16_t* absum, int M,
                                                       int M_stride, int ash, int Mp, int K, uint8_t* af, uint32_t* u) {
   const int nb = K / 32;
@@ -68,7 +74,7 @@ __global__ __launch_bounds__(256) void f16_act_kernel(const int8_t* aq, const fl
   uint32_t hw[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (m < M) {
     const int8_t* src = aq + (size_t)m * K + 32 * b;
-    const uint2 q0 = *(const uint2*)(src + 8 * h), q1 = *(const uint2*)(src + 16 + 8 * h);
+    const uint2 q0 = *(const uint2*)(src + (HALF ? 16 : 8) * h), q1 = *(const uint2*)(src + (HALF ? 8 + 16 * h : 16 + 8 * h));
     const uint32_t qw[4] = {q0.x, q0.y, q1.x, q1.y};
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -77,7 +83,7 @@ __global__ __launch_bounds__(256) void f16_act_kernel(const int8_t* aq, const fl
         uint32_t pr = 0;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          const int e = f16_perm8(i + t);  // element 16c + 8h + e
+          const int e = f16_perm8(i + t);  // element 16c + 8h + e (HALF: 16h + 8c + e)
           const int8_t qv = (int8_t)(qw[2 * c + (e >> 2)] >> (8 * (e & 3)));
           pr |= (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)qv) << (16 * t);
         }
@@ -153,6 +159,72 @@ __device__ __forceinline__ void q4k_f16_decode(uint32_t x, uint32_t y, int sc, u
   }
 }
 
+// A lane's share of a 32-block: Q4_K its 8 nibble bytes (x y); Q5_K the 8 nibble bytes of its half and the word of fifth bits
+// (z); IQ3_S the four index bytes of its half (x) and the block's sign bytes (y)
+struct F16Pay {
+  uint32_t x, y, z;
+};
+template <int TYPE>
+__device__ __forceinline__ F16Pay f16_load(const uint8_t* qrow, int blk, int h) {
+  const uint8_t* r = qrow + (size_t)blk * Traits<TYPE>::QB;
+  if constexpr (TYPE == T_IQ3_S) {
+    return F16Pay{*(const uint32_t*)(r + 4 * h), *(const uint32_t*)(r + 8), 0u};
+  } else {
+    const uint2 v = *(const uint2*)(r + 8 * h);
+    return F16Pay{v.x, v.y, TYPE == T_Q5_K ? *(const uint32_t*)(r + 16) : 0u};
+  }
+}
+
+// Block b (0..7) of a superblock with header hdr: the lane's 16 values times the integer block scale, as the two f16 operands
+template <int TYPE>
+__device__ __forceinline__ void f16_decode(const F16Pay& p, uint4 hdr, int b, int h, const typename LdsFor<TYPE>::type* tab,
+                                           f16x8& b0, f16x8& b1) {
+  if constexpr (TYPE == T_Q4_K) {
+    int sc, mn;
+    q4k_scale_min(hdr.y, hdr.z, hdr.w, b, sc, mn);
+    (void)mn;
+    q4k_f16_decode(p.x, p.y, sc, 0x64006400u, b0, b1);
+  } else {
+    // words w[k] of bytes u (elements 16h + 4k ..): (1024 + u) as f16 is 0x6400 | u, and (1024 + u) sc - (1024 + bias) sc is
+    // exact as in q4k_f16_decode (bias 128 takes IQ3_S's signed bytes, flipped to unsigned, back)
+    uint32_t w[4];
+    int sc;
+    if constexpr (TYPE == T_Q5_K) {
+      int mn;
+      q4k_scale_min(hdr.y, hdr.z, hdr.w, b, sc, mn);
+      (void)mn;
+      const uint32_t hb = p.z >> (4 * h);
+      w[0] = (p.x & 0x0F0F0F0Fu) | ((hb & 0x01010101u) << 4);
+      w[1] = (p.y & 0x0F0F0F0Fu) | ((hb & 0x02020202u) << 3);
+      w[2] = ((p.x >> 4) & 0x0F0F0F0Fu) | ((hb & 0x04040404u) << 2);
+      w[3] = ((p.y >> 4) & 0x0F0F0F0Fu) | ((hb & 0x08080808u) << 1);
+    } else {
+      const uint32_t qh = ((b < 4 ? hdr.x : hdr.y) >> (8 * (b & 3) + 4 * h)) & 0xFu, sg = p.y >> (16 * h);
+      sc = 1 + 2 * (int)((hdr.z >> (4 * b)) & 0xFu);
+      const uint4 m0 = tab->sgn[sg & 0xFFu], m1 = tab->sgn[(sg >> 8) & 0xFFu];
+      w[0] = (tab->grid[(p.x & 0xFFu) | ((qh << 8) & 256u)] ^ m0.x) + m0.z;
+      w[1] = (tab->grid[((p.x >> 8) & 0xFFu) | ((qh << 7) & 256u)] ^ m0.y) + m0.w;
+      w[2] = (tab->grid[((p.x >> 16) & 0xFFu) | ((qh << 6) & 256u)] ^ m1.x) + m1.z;
+      w[3] = (tab->grid[(p.x >> 24) | ((qh << 5) & 256u)] ^ m1.y) + m1.w;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) w[k] ^= 0x80808080u;
+    }
+    const _Float16 s = (_Float16)sc, o = (_Float16)(TYPE == T_IQ3_S ? -1152.0f : -1024.0f) * s;
+    const f16x2 sc2 = {s, s}, off2 = {o, o};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const f16x2 v0 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, w[k], 0x04020400u)) * sc2 + off2;
+      const f16x2 v1 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, w[k], 0x04030401u)) * sc2 + off2;
+      f16x8& d = k < 2 ? b0 : b1;
+      const int i = 4 * (k & 1);
+      d[i] = v0[0];
+      d[i + 1] = v0[1];
+      d[i + 2] = v1[0];
+      d[i + 3] = v1[1];
+    }
+  }
+}
+
 // Work-group -> (128-row weight tile, 128-token tile, K piece); consecutive work-groups of one XCD (work-groups are dealt to
 // the 8 XCDs round-robin) take neighbouring weight tiles of one token tile, so the token tile stays in that XCD's L2.
 // Returns the index of the piece among the cut tiles' pieces, or -1 for a whole tile.
@@ -192,10 +264,13 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
   const int n_rows = a.w.rows;
   const int nbase = nt * kF16BN + wave * 32;
   const int nrow = min(nbase + lc, n_rows - 1);  // this lane's A-operand row
-  const uint8_t* qrow = a.w.qs + (size_t)nrow * nb * 16 + 8 * h;
+  constexpr bool MINS = Traits<TYPE>::MINS;
+  static_assert(Traits<TYPE>::HB == 16, "16-byte headers");
+  __shared__ typename LdsFor<TYPE>::type tab;
+  lds_fill<TYPE>(&tab);
+  const uint8_t* qrow = a.w.qs + (size_t)nrow * nb * Traits<TYPE>::QB;
   const uint8_t* hrow = a.w.hdr + (size_t)nrow * nsb * 16;
   const uint8_t* abase = a.af + (size_t)mt * npair * kF16PairBytes;
-  const uint32_t c64 = 0x64006400u;
 
   // activation staging: 16 KB per block pair, 4 x 16 bytes per thread
   u32x4_t st[4];
@@ -227,9 +302,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
   const f32x16 zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
   uint4 hdr = *(const uint4*)(hrow + (size_t)sb0 * 16), hdr_n;
-  uint2 pay[2], pay_n[2];
+  F16Pay pay[2], pay_n[2];
 #pragma unroll
-  for (int bb = 0; bb < 2; ++bb) pay[bb] = *(const uint2*)(qrow + (size_t)(8 * sb0 + bb) * 16);
+  for (int bb = 0; bb < 2; ++bb) pay[bb] = f16_load<TYPE>(qrow, 8 * sb0 + bb, h);
   fetch_sa(4 * sb0);
   fetch(4 * sb0);
   store(0);
@@ -245,18 +320,13 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
       const int gn = g + 1 < 4 * sb1 ? g + 1 : g;
       fetch(gn);
 #pragma unroll
-      for (int bb = 0; bb < 2; ++bb) pay_n[bb] = *(const uint2*)(qrow + (size_t)(2 * gn + bb) * 16);
+      for (int bb = 0; bb < 2; ++bb) pay_n[bb] = f16_load<TYPE>(qrow, 2 * gn + bb, h);
       fetch_sa(gn);
       // (keeps the loads here: issued a whole pair of MFMA work before their data is needed)
       __builtin_amdgcn_sched_barrier(0);
       f16x8 aw[2][2];
 #pragma unroll
-      for (int bb = 0; bb < 2; ++bb) {
-        int sc, mn;
-        q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * p + bb, sc, mn);
-        (void)mn;
-        q4k_f16_decode(pay[bb].x, pay[bb].y, sc, c64, aw[bb][0], aw[bb][1]);
-      }
+      for (int bb = 0; bb < 2; ++bb) f16_decode<TYPE>(pay[bb], hdr, 2 * p + bb, h, &tab, aw[bb][0], aw[bb][1]);
       const uint8_t* L = lds + cur * kF16PairBytes + lane * 16;
       if constexpr (S256) {
         // items block-major (k = 4 bb + t): consecutive MFMAs feed different token tiles' accumulators
@@ -352,14 +422,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
       // superblock epilogue: res = fma(d, tq, fma(-dmin, tmn, res)) (gemm.cl:395-398). d and dmin are per weight row,
       // i.e. per result register: each lane publishes its row's pair in LDS and reads those of its 16 rows.
       if (h == 0) {
-        dtab[wave][0][lc] = h2f(hdr.x);
-        dtab[wave][1][lc] = h2f(hdr.x >> 16);
+        dtab[wave][0][lc] = h2f(TYPE == T_IQ3_S ? hdr.w : hdr.x);
+        if constexpr (MINS) dtab[wave][1][lc] = h2f(hdr.x >> 16);
       }
       int mn[8];
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
         int scv;
-        q4k_scale_min(hdr.y, hdr.z, hdr.w, b, scv, mn[b]);
+        if constexpr (MINS) q4k_scale_min(hdr.y, hdr.z, hdr.w, b, scv, mn[b]);
+        else mn[b] = 0;
       }
       // mins operand (A: weight rows): slot 8h + i = mn of block 4h + i / 2 (a bit select on the two candidates: a
       // lane-dependent array index would put mn in scratch memory)
@@ -371,12 +442,20 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float4 dv = *(const float4*)&dtab[wave][0][8 * q + 4 * h];
-        const float4 mv = *(const float4*)&dtab[wave][1][8 * q + 4 * h];
         dr[4 * q] = dv.x; dr[4 * q + 1] = dv.y; dr[4 * q + 2] = dv.z; dr[4 * q + 3] = dv.w;
-        dmr[4 * q] = -mv.x; dmr[4 * q + 1] = -mv.y; dmr[4 * q + 2] = -mv.z; dmr[4 * q + 3] = -mv.w;
+        if constexpr (MINS) {
+          const float4 mv = *(const float4*)&dtab[wave][1][8 * q + 4 * h];
+          dmr[4 * q] = -mv.x; dmr[4 * q + 1] = -mv.y; dmr[4 * q + 2] = -mv.z; dmr[4 * q + 3] = -mv.w;
+        }
       }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
+        if constexpr (!MINS) {
+          const float sv = S256 ? sv256[t] : 1.0f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) res[t][r] = fmaf(S256 ? dr[r] * sv : dr[r], tq[t][r], res[t][r]);
+          continue;
+        }
         const uint4 uv = *(const uint4*)(a.u + (size_t)(m0 + 32 * t + lc) * nb + 8 * s + 4 * h);
         const f32x16 tmn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mnop, __builtin_bit_cast(bf16x8, uv), zero16, 0, 0, 0);
         if constexpr (S256) {
@@ -428,9 +507,19 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
 
 // ---- host side
 
-bool f16_gemm_supported(int type, int M, int K) {
-  if (type != T_Q4_K) return false;
-  return M >= 128 && K % 256 == 0;
+// Q4_K: every prompt of 128 tokens and more. Q5_K and IQ3_S, whose int8 kernels run without a workspace: where the product
+// is long enough for the call to wait for the GPU (the workspace costs the host about 20 us), 128-token tiles waste at most a
+// fifth of their rows, and the tiles' time here, with the prepass's, is under the int8 kernel's by the two kernels' measured rates
+// (microseconds of a round's superblock: Q5_K 7.4 against 4.5 for half the tiles' size, IQ3_S 7.2 against 4.0; 2048 x 5120 -> 17408
+// Q5_K 771 -> 660 us, IQ3_S 695 -> 650; 512 x 5120 -> 5120 86.6 -> 72.7 and 79.3 -> 70.3; but 1024 x 4096 -> 4096, 256 tiles here
+// and 512 there, 86.7 against 79.7 and 84.7 against 71.9).
+bool f16_gemm_supported(int type, int M, int rows, int K) {
+  if (M < 128 || K % 256) return false;
+  if (type == T_Q4_K) return true;
+  if (type != T_Q5_K && type != T_IQ3_S) return false;
+  if ((double)M * rows * K < 1.2e10 || round_up((size_t)M, kF16BM) * 4 > (size_t)M * 5) return false;
+  const float here = gemm_split_for(type, M, rows, K, true).cost * (type == T_Q5_K ? 7.4f : 7.2f) + (float)M * (float)K * 1e-6f;
+  return here < 0.97f * gemm_split_for(type, M, rows, K, false).cost * (type == T_Q5_K ? 4.5f : 4.0f);
 }
 
 // One memory pool per device for the per-call workspace (stream-ordered: concurrent calls on different streams get
@@ -496,8 +585,9 @@ hipError_t f16_scratch(void** out, size_t* bytes, void** part) {
   return hipSuccess;
 }
 
-hipError_t launch_gemm_f16(int type, const GemmArgs& g, void* ws, hipStream_t s) {
-  if (type != T_Q4_K) return hipErrorInvalidValue;
+template <int TYPE>
+static hipError_t go_f16(const GemmArgs& g, void* ws, hipStream_t s) {
+  constexpr bool MINS = Traits<TYPE>::MINS, HALF = kF16Half<TYPE>;
   const int M = g.M, K = g.w.K;
   const int Mp = (int)round_up((size_t)M, kF16BM);
   void* buf = ws;
@@ -511,10 +601,10 @@ hipError_t launch_gemm_f16(int type, const GemmArgs& g, void* ws, hipStream_t s)
   const size_t threads = (size_t)Mp * (K / 32) * 2;
   // (the block-sum mode reads no activation scales: no mins operand)
   if (g.dbg_isum)
-    f16_act_kernel<false><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(g.aq, nullptr, nullptr, M,
+    f16_act_kernel<false, HALF><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(g.aq, nullptr, nullptr, M,
                                                                                        g.M_stride, 0, Mp, K, af, u);
   else
-    f16_act_kernel<true><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(g.aq, g.asc, g.absum, M,
+    f16_act_kernel<MINS, HALF><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(g.aq, g.asc, g.absum, M,
                                                                                       g.M_stride, g.ash, Mp, K, af, u);
   e = hipGetLastError();
   if (e == hipSuccess) {
@@ -536,11 +626,11 @@ hipError_t launch_gemm_f16(int type, const GemmArgs& g, void* ws, hipStream_t s)
     a.splits = g.splits;
     const int gx = (g.w.rows + kF16BN - 1) / kF16BN, gy = Mp / kF16BM, tiles = gx * gy;
     const dim3 grid((unsigned)(g.part ? g.split_from + (tiles - g.split_from) * g.splits : tiles));
-    if (g.dbg_isum) gemm_f16_kernel<T_Q4_K, true><<<grid, dim3(256), 0, s>>>(a);
-    else if (g.ash == 3 && g.part) gemm_f16_kernel<T_Q4_K, false, true, true><<<grid, dim3(256), 0, s>>>(a);
-    else if (g.ash == 3) gemm_f16_kernel<T_Q4_K, false, true><<<grid, dim3(256), 0, s>>>(a);
-    else if (g.part) gemm_f16_kernel<T_Q4_K, false, false, true><<<grid, dim3(256), 0, s>>>(a);
-    else gemm_f16_kernel<T_Q4_K, false><<<grid, dim3(256), 0, s>>>(a);
+    if (g.dbg_isum) gemm_f16_kernel<TYPE, true><<<grid, dim3(256), 0, s>>>(a);
+    else if (g.ash == 3 && g.part) gemm_f16_kernel<TYPE, false, true, true><<<grid, dim3(256), 0, s>>>(a);
+    else if (g.ash == 3) gemm_f16_kernel<TYPE, false, true><<<grid, dim3(256), 0, s>>>(a);
+    else if (g.part) gemm_f16_kernel<TYPE, false, false, true><<<grid, dim3(256), 0, s>>>(a);
+    else gemm_f16_kernel<TYPE, false><<<grid, dim3(256), 0, s>>>(a);
     e = hipGetLastError();
     if (e == hipSuccess && g.part) e = launch_split_sum(g, kF16BM, tiles, gx, gy, false, s);
   }
@@ -549,6 +639,15 @@ hipError_t launch_gemm_f16(int type, const GemmArgs& g, void* ws, hipStream_t s)
     if (e == hipSuccess) e = e2;
   }
   return e;
+}
+
+hipError_t launch_gemm_f16(int type, const GemmArgs& g, void* ws, hipStream_t s) {
+  switch (type) {
+    case T_Q4_K: return go_f16<T_Q4_K>(g, ws, s);
+    case T_Q5_K: return go_f16<T_Q5_K>(g, ws, s);
+    case T_IQ3_S: return go_f16<T_IQ3_S>(g, ws, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace qm

@@ -88,42 +88,47 @@ constexpr size_t kSplitBytes = (size_t)32 << 20;  // most partial tiles of one c
 struct GemmSplit {
   int from, splits;  // tiles [0, from) whole, [from, tiles) in `splits` pieces each (splits = 1: none)
   size_t bytes;      // partial tiles
+  bool halves;       // uncut, two K halves added into a zeroed C
+  float cost;        // the call's time in superblocks of a full round
 };
 // Rounds that n equal work-groups take; alone: the time of a round that fills half the slots or less (a work-group that has
-// its CU to itself runs faster than two that share it), as a part of a full one
+// its CU to itself runs faster than two that share it), as a part of a full one. Many rounds overlap and cost their share.
 inline float gemm_rounds(int n, float alone) {
   const int rem = n % kGemmSlots;
+  if (n > 2 * kGemmSlots) return (float)n / kGemmSlots;
   return (float)(n / kGemmSlots) + (rem == 0 ? 0.0f : 2 * rem <= kGemmSlots ? alone : 1.0f);
 }
 // tiles of bm x 128 results, K of nsb superblocks; us: microseconds of a full round's superblock; host: those below which the
-// call would wait for its own workspace (0: it has one anyway); halves: uncut, a small product's two K halves are added into a zeroed C.
-// With more than one whole round the last one starts while others still run, and cutting it measured level (Q4_K 2048 x 5120 ->
-// 17408, 2176 tiles: 572 us either way), so only products of fewer than 1024 tiles are cut.
+// call would wait for its own workspace (0: it has one anyway); halves: a small product may add two K halves into a zeroed C.
+// A work-group costs its superblocks and about one more (its prologue and store). With more than one whole round the last one
+// starts while others still run, and cutting it measured level (Q4_K 2048 x 5120 -> 17408, 2176 tiles: 572 us either way), so
+// only products of fewer than 1024 tiles are cut, of K 2048 and more, for a tenth or more.
 inline GemmSplit gemm_split(int tiles, int nsb, int bm, bool halves, float alone, float us, float host) {
-  GemmSplit r{tiles, 1, 0};
+  GemmSplit r{tiles, 1, 0, false, gemm_rounds(tiles, alone) * (float)(nsb + 1)};
   const int full = tiles / kGemmSlots * kGemmSlots, rem = tiles - full;
-  if (rem == 0 || full > kGemmSlots) return r;
-  // time of the tail in superblocks per slot: a piece costs its superblocks and about one more (its prologue and store), the
-  // second kernel about 1.5 and the partial tiles' traffic 1.4 per 512 pieces of 64 x 128 results. Cut for a tenth or more.
-  float best = gemm_rounds(rem, alone) * (float)nsb;
-  if (halves && tiles < kGemmSlots && nsb >= 8) best = fminf(best, gemm_rounds(2 * rem, alone) * (float)(nsb / 2 + 1) + 2.0f);
-  const float uncut = (best + (float)(full / kGemmSlots * nsb)) * us;
-  best = 0.9f * best;
+  if (halves && nsb >= 8 && tiles < kGemmSlots) {
+    const float t = gemm_rounds(2 * tiles, alone) * (float)(nsb / 2 + 1) + 3.0f;  // (3: zeroing C, adding into it)
+    // (up to one tile per CU always: IQ4_XS 333 x 17408 -> 5120, 240 tiles, 131 us in halves against 156, 200 x 5120 -> 5120, 160
+    //  tiles, 45 against 51; above, when the doubled grid does not take as many rounds)
+    if (2 * tiles <= kGemmSlots || t < r.cost) {
+      r.cost = t;
+      r.halves = true;
+    }
+  }
+  if (rem == 0 || full > kGemmSlots || nsb < 8) return r;
+  const float uncut = r.cost, whole = (float)(full / kGemmSlots) * (float)(nsb + 1);
   for (int s = 2; s <= 8 && nsb / s >= 2; ++s) {
     const size_t bytes = (size_t)rem * s * bm * 128 * sizeof(float);
-    const float t = gemm_rounds(rem * s, alone) * ((float)((nsb + s - 1) / s) + 1.0f) + 1.5f +
-                    1.4f * (float)(rem * s) * (float)bm / (64.0f * 512.0f);
-    const float cut = (t + (float)(full / kGemmSlots * nsb)) * us;
-    if (host > 0.0f && uncut - fmaxf(cut, host) < 8.0f) continue;
-    if (t < best && bytes <= kSplitBytes) {
-      best = t;
-      r = GemmSplit{full, s, bytes};
-    }
+    // (the second kernel about 0.7, the partial tiles' traffic 0.7 per 512 pieces of 64 x 128 results)
+    const float t = whole + gemm_rounds(rem * s, alone) * (float)((nsb + s - 1) / s + 1) + 0.7f +
+                    0.7f * (float)(rem * s) * (float)bm / (64.0f * 512.0f);
+    if (host > 0.0f && (uncut - fmaxf(t, host / us)) * us < 8.0f) continue;
+    if (t < r.cost && t < 0.9f * uncut && bytes <= kSplitBytes) r = GemmSplit{full, s, bytes, r.halves, t};
   }
   return r;
 }
-// The same for one call: the kernel that launch_gemm / launch_gemm_f16 takes for it (splits = 1 where it takes another)
-GemmSplit gemm_split_for(int type, int M, int rows, int K);
+// The same for one call, on the f16 path or by launch_gemm (splits = 1 where that takes the few-token kernels)
+GemmSplit gemm_split_for(int type, int M, int rows, int K, bool f16);
 // C (op)= the sums of the cut tiles' pieces (bm x 128 each); tile t: rows bm * (t % gy).., columns 128 * (t / gy).. when
 // m_fast, else bm * (t / gx).., 128 * (t % gx)..
 hipError_t launch_split_sum(const GemmArgs& a, int bm, int tiles, int gx, int gy, bool m_fast, hipStream_t s);
@@ -134,7 +139,7 @@ enum GemmMode : int { GEMM_DENSE = 0, GEMM_MOE_GATEUP = 1, GEMM_MOE_DOWN = 2, GE
 hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s);
 // Prompt GEMM on the f16 matrix pipe (qm_gemm_f16.hip): the types and shapes it takes, its per-call workspace, and
 // the launcher (ws = null: the workspace comes from a per-device stream-ordered pool). dbg_isum: block-sum mode.
-bool f16_gemm_supported(int type, int M, int K);
+bool f16_gemm_supported(int type, int M, int rows, int K);
 size_t f16_workspace_bytes(int M, int K);
 hipError_t launch_gemm_f16(int type, const GemmArgs& a, void* ws, hipStream_t s);
 // The current device's copies of the static scratch arrays for the allocation-free entry: ptr (bytes) the f16 path's

@@ -76,3 +76,33 @@ def test_captured_call_matches(qm, dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(C, want)
+
+
+@pytest.mark.parametrize("qtype", [F.Q5_K, F.IQ3_S])
+@pytest.mark.parametrize("act32", [True, False])
+def test_f16_types(qm, dev, qtype, act32):
+    """Q5_K and IQ3_S products long enough for the f16 kernels (ragged rows and tokens, whole and cut tiles): f32 parity, block
+    sums bit for bit, and the int8 kernels behind the same call without a workspace."""
+    import torch
+    M, N, K = 500, 4624, 5376
+    W = F.synth_weight(qtype, N, K, seed=qtype)
+    x = F.synth_activations(M, K, seed=K, outlier_frac=0.01)
+    aq, asc, absum = qm.quantize_act(to_dev(x, dev), M_stride=M + 3, act32=act32)
+    w = qm.QWeight(qtype, to_dev(W, dev), N, K)
+    assert qm.gemm_workspace_size(w, M) > 2 * M * K
+    C = qm.gemm(w, aq, asc, absum, M=M, act32=act32)
+    D = qm.gemm_ws(w, aq, asc, absum, None, M=M, act32=act32)
+    torch.cuda.synchronize()
+    stride = 37
+    blockdot = oracle.blockdot if act32 else oracle.blockdot256
+    ref = blockdot(qtype, W, K, aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy(), M=M, col_stride=stride)
+    sel = np.arange(0, N, stride)
+    ref = ref[:, sel] if ref.shape[1] == N else ref
+    for got in (C, D):
+        assert rel_err(got.cpu().numpy()[:, sel], ref) < TOL_INT8_PATH
+        assert_elementwise(got.cpu().numpy()[:, sel], ref)
+    if act32:
+        R = 64  # (rows of the block sums; the kernel choice follows the whole product's shape, so the full matrix is run)
+        isum = qm.gemm_blocksums(w, aq, M=M)[:, :R].cpu().numpy()
+        _, risum, _ = oracle.blockdot(qtype, W[:R], K, aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy(), M=M, blocksums=True)
+        assert np.array_equal(isum, risum)
