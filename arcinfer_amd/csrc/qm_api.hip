@@ -5,6 +5,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 
 #include "../../include/qmatmul.h"
@@ -75,6 +76,8 @@ size_t plane_qs_bytes(int t, int rows, int K) { return (size_t)rows * (K / 32) *
 size_t plane_hdr_bytes(int t, int rows, int K) { return (size_t)rows * (K / 256) * header_bytes(t); }
 
 bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
+
+std::atomic<int> g_weights{0};  // prepared weights that are not released yet
 
 std::once_flag g_init_once;
 int g_init_status = QM_OK;
@@ -239,6 +242,7 @@ int qmatmul_prepare_weight(int type, const void* raw, int raw_on_device, int row
     delete w;
     return hip_fail(e, "qmatmul_prepare_weight: repack");
   }
+  g_weights.fetch_add(1);
   *out = w;
   return QM_OK;
 }
@@ -247,6 +251,7 @@ int qmatmul_release_weight(qm_weight* w) {
   if (!w) return fail(QM_ERR_ARG, "qmatmul_release_weight: null weight");
   hipError_t e = hipFree(w->base);
   delete w;
+  if (g_weights.fetch_sub(1) == 1) qm::workspaces_give_back();
   if (e != hipSuccess) return hip_fail(e, "qmatmul_release_weight: hipFree");
   return QM_OK;
 }
@@ -455,7 +460,7 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   size_t need = f16 ? align256(fb) : 0;
   qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, K, f16);
   size_t pb = sp.splits > 1 ? sp.bytes : 0;  // partial tiles (optional)
-  void* pool = nullptr;
+  qm::CallWs call;
   float* part = nullptr;
   if (wm == WS_STATIC) {
     if (pb) part = (float*)static_part;
@@ -464,15 +469,15 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   } else {
     if (capturing) pb = 0;
     if (need + pb) {
-      e = qm::pool_alloc(&pool, need + pb, (hipStream_t)stream);
+      e = qm::workspace_take(&call, need + pb, capturing, (hipStream_t)stream);
       if (e == hipSuccess) {
-        if (f16) scr = pool;
-        if (pb) part = (float*)((uint8_t*)pool + need);
+        if (f16) scr = call.p;
+        if (pb) part = (float*)((uint8_t*)call.p + need);
       } else if (w->type == QM_Q4_K && f16) {
         return hip_fail(e, fn);
       } else {
         (void)hipGetLastError();  // (no memory: the int8 kernels, uncut, need none)
-        pool = nullptr;
+        call.p = nullptr;
         f16 = false;
       }
     }
@@ -484,8 +489,8 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   }
   e = f16 ? qm::launch_gemm_f16(w->type, a, scr, (hipStream_t)stream)
           : qm::launch_gemm(w->type, qm::GEMM_DENSE, a, (hipStream_t)stream);
-  if (pool) {
-    const hipError_t e2 = hipFreeAsync(pool, (hipStream_t)stream);
+  if (call.p) {
+    const hipError_t e2 = qm::workspace_done(call, (hipStream_t)stream);
     if (e == hipSuccess) e = e2;
   }
   return e == hipSuccess ? QM_OK : hip_fail(e, fn);

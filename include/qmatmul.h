@@ -144,11 +144,13 @@ int qmatmul_gemv(const qm_weight* w, const int8_t* aq, const float* asc, const i
 /* Prompt GEMM: C[m*ldc + c_off + n] (op)= sum_k W[n][k] * a_m[k] for m < M.
  * M <= M_stride; any M >= 1 and rows(w) % 16 == 0. Replaces decode_w8 + gemm of Engine::matmul1 for T > 8 and
  * gemm_ext (zero/engine.h:3234-3297; zero/kernels/gemm.cl:132-475). Q4_K is computed exactly (scales and mins),
- * not requantized as the reference's W8 path does (zero/kernels/decode.cl:455-507). Q4_K with M >= 128 runs on the
- * f16 matrix pipe (exact integer block sums from f16 products) and takes a per-call workspace of about 2*M*K bytes
- * from a per-device stream-ordered memory pool; every other case runs on int8 MFMA. Products of few tiles, or of few more
- * than the chip holds at once, are cut along K and take up to 32 MiB of that pool for the pieces' partial results (not on a
- * stream under capture, nor when the pool has none: they then run uncut, equal up to f32 rounding order). A caller
+ * not requantized as the reference's W8 path does (zero/kernels/decode.cl:455-507). Q4_K with M >= 128, and longer products of
+ * Q5_K and IQ3_S, run on the f16 matrix pipe (exact integer block sums from f16 products) with a per-call workspace of about
+ * 2*M*K bytes; products of few tiles, or of few more than the chip holds at once, are cut along K and take up to 32 MiB for the
+ * pieces' partial results; every other case runs on int8 MFMA without. The workspace is one of a few buffers kept between
+ * calls (at most 8 of 128 MiB a device, returned when the last weight is released; calls on any streams and threads may
+ * overlap) or memory of a per-device stream-ordered pool. On a stream under capture only Q4_K takes one (the pool's); the others
+ * then run uncut on int8 MFMA, equal up to f32 rounding order, as they do when there is no memory. A caller
  * that owns all memory passes the workspace itself (qmatmul_gemm_ws). */
 int qmatmul_gemm(const qm_weight* w, const int8_t* aq, const float* asc, const int16_t* absum, int M, int M_stride,
                  float* C, int ldc, int c_off, int accumulate, void* stream);

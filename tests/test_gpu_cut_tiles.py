@@ -106,3 +106,42 @@ def test_f16_types(qm, dev, qtype, act32):
         isum = qm.gemm_blocksums(w, aq, M=M)[:, :R].cpu().numpy()
         _, risum, _ = oracle.blockdot(qtype, W[:R], K, aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy(), M=M, blocksums=True)
         assert np.array_equal(isum, risum)
+
+
+def test_kept_workspaces_over_streams_and_threads(qm, dev):
+    """More streams than kept workspaces, each with its own inputs, calls in turn and from threads: every result is the one of a
+    call by itself; and again after the last weight (of this test) went and came back."""
+    import threading
+
+    import torch
+    M, N, K, S = 130, 144, 2048, 11
+    W = to_dev(F.synth_weight(F.Q4_K, N, K, seed=5), dev)
+    xs = [acts(qm, F.synth_activations(M, K, seed=100 + i), dev, M_stride=M) for i in range(S)]
+    for _ in range(2):
+        w = qm.QWeight(F.Q4_K, W, N, K)
+        want = [qm.gemm(w, *x, M=M) for x in xs]
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream() for _ in range(S)]
+        out = [[torch.empty((M, N), device=dev) for _ in range(4)] for _ in range(S)]
+        torch.cuda.synchronize()
+
+        def calls(i):
+            for C in out[i]:
+                qm.gemm(w, *xs[i], M=M, C=C, ldc=N, stream=streams[i].cuda_stream)
+
+        for i in range(S):
+            calls(i)
+        torch.cuda.synchronize()
+        assert all(torch.equal(C, want[i]) for i in range(S) for C in out[i])
+        for i in range(S):
+            for C in out[i]:
+                C.zero_()
+        torch.cuda.synchronize()
+        ts = [threading.Thread(target=calls, args=(i,)) for i in range(S)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        torch.cuda.synchronize()
+        assert all(torch.equal(C, want[i]) for i in range(S) for C in out[i])
+        w.release()
