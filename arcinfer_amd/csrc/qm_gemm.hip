@@ -1108,9 +1108,22 @@ static hipError_t go(const GemmArgs& a, hipStream_t s) {
   }
 }
 
+// Four row tiles per work-group share each decoded operand where the decode is a codebook lookup (a third of the VALU work at
+// two tiles) and 128-token tiles still make two and a half rounds of work-groups with little padding: IQ4_XS 2048 x 5120 -> 17408
+// 645 -> 600 us, 4096 x 5120 -> 5120 (1280 tiles) 380 -> 354; 1024 x 5120 -> 17408 (1088 tiles) 331 -> 337. (Q8_0, which decodes nothing: 570 either way.)
+template <int TYPE>
+static bool four_row_tiles(const GemmArgs& a) {
+  if (TYPE != T_IQ4_XS && TYPE != T_IQ4_NL) return false;
+  const int gy = (a.M + 127) / 128;
+  return (a.w.rows + 127) / 128 * gy >= 5 * kGemmSlots / 2 && gy * 128 * 16 <= a.M * 17;
+}
+
 template <int TYPE>
 static hipError_t dispatch(int mode, const GemmArgs& a, hipStream_t s) {
   // (the block-sum mode takes the product's row-tile count, so the sums checked are those of the kernel that runs)
+  if constexpr (TYPE == T_IQ4_XS || TYPE == T_IQ4_NL)
+    if (mode == GEMM_DENSE && four_row_tiles<TYPE>(a))
+      return a.dbg_isum ? go<TYPE, 4, GEMM_DENSE, true>(a, s) : go<TYPE, 4, GEMM_DENSE, false>(a, s);
   if (a.dbg_isum) return a.M <= 32 ? go<TYPE, 1, GEMM_DENSE, true>(a, s) : go<TYPE, 2, GEMM_DENSE, true>(a, s);
   switch (mode) {
     case GEMM_DENSE:

@@ -145,3 +145,22 @@ def test_kept_workspaces_over_streams_and_threads(qm, dev):
         torch.cuda.synchronize()
         assert all(torch.equal(C, want[i]) for i in range(S) for C in out[i])
         w.release()
+
+
+@pytest.mark.parametrize("qtype", [F.IQ4_XS, F.IQ4_NL])
+def test_four_row_tiles(qm, dev, qtype):
+    """Products of 1280 tiles of 128 x 128 and more (four row tiles per work-group for these types), the last row and column
+    tile ragged: parity on sampled columns, block sums bit for bit on the first and last rows."""
+    import torch
+    M, N, K = 2047, 10256, 256
+    W = F.synth_weight(qtype, N, K, seed=qtype)
+    aq, asc, absum = acts(qm, F.synth_activations(M, K, seed=3, outlier_frac=0.01), dev, M_stride=2048)
+    w = qm.QWeight(qtype, to_dev(W, dev), N, K)
+    C = qm.gemm(w, aq, asc, absum, M=M).cpu().numpy()
+    isum = qm.gemm_blocksums(w, aq, M=M)
+    a = (aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy())
+    for r in (slice(0, 32), slice(N - 32, N)):
+        ref, risum, _ = oracle.blockdot(qtype, W[r], K, *a, M=M, blocksums=True)
+        assert rel_err(C[:, r], ref) < TOL_INT8_PATH
+        assert_elementwise(C[:, r], ref)
+        assert np.array_equal(isum[:, r].cpu().numpy(), risum)
