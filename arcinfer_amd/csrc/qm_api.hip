@@ -443,7 +443,7 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   }
   // the f16 path's activations: Q4_K must have room for them; the other types of that path run on int8 MFMA without (and on a
   // capturing stream, where they record no allocation)
-  const size_t fb = qm::f16_workspace_bytes(M, K);
+  const size_t fb = qm::f16_workspace_bytes(w->type, M, K);
   bool f16 = qm::f16_gemm_supported(w->type, M, w->rows, K);
   if (f16 && w->type != QM_Q4_K)
     f16 = wm == WS_STATIC ? fb <= cap_bytes : wm == WS_CALLER ? ws && ws_bytes >= fb && aligned(ws, 256) : !capturing;
@@ -511,7 +511,7 @@ int qmatmul_gemm_ex(const qm_weight* w, const int8_t* aq, const float* asc, cons
 size_t qmatmul_gemm_workspace_size(const qm_weight* w, int M) {
   if (!w || M < 1) return 0;
   const bool f16 = qm::f16_gemm_supported(w->type, M, w->rows, w->view.K);
-  const size_t need = f16 ? qm::f16_workspace_bytes(M, w->view.K) : 0;
+  const size_t need = f16 ? qm::f16_workspace_bytes(w->type, M, w->view.K) : 0;
   const qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, w->view.K, f16);
   return sp.splits > 1 ? align256(need) + sp.bytes : need;
 }

@@ -10,7 +10,7 @@
 // (|I| <= 32 * 127 * 945 < 2^24) is the exact integer. The per-block activation scale is then applied with one f32 fma
 // per element, as the reference does; with tokens on the MFMA's columns, asc is one value per lane. tmn is one bf16
 // MFMA per superblock (asc * bsum split into two bf16 parts, 16 bits; mn exact), and d, dmin are applied once per
-// superblock in the reference's order.
+// superblock in the reference's order. Q5_K: kF16Centred.
 //
 // Work-group: 4 waves, a tile of 128 weight rows x 128 tokens; wave w owns weight rows 32w..32w+31 (one MFMA row
 // tile, decoded once per block in registers) for all 128 tokens (four 32-token column tiles). Two work-groups per CU,
@@ -44,27 +44,39 @@ __host__ __device__ constexpr int f16_perm8(int i) { return (i & 4) | ((i & 1) <
 
 static size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
-// Workspace of one call (device bytes), for M tokens and K columns: the f16 activations, then the mins operand.
-size_t f16_workspace_bytes(int M, int K) {
+// Workspace of one call (device bytes), for M tokens and K columns: the f16 activations, then the mins operand (Q5_K: twice,
+// kF16Centred).
+size_t f16_workspace_bytes(int type, int M, int K) {
   const size_t Mp = round_up((size_t)M, kF16BM);
-  return round_up(Mp * (size_t)K * 2, 256) + Mp * (size_t)(K / 32) * 4;
+  return round_up(Mp * (size_t)K * 2, 256) + Mp * (size_t)(K / 32) * (type == T_Q5_K ? 8 : 4);
 }
 
 // The types of this kernel: Q4_K (Q5_K's and IQ3_S's values times their integer block scales fit an f16 exactly too: 31 * 63 =
 // 1953, 15 * 31 = 465). kF16Half: see f16_act_kernel.
 template <int TYPE> constexpr bool kF16Half = TYPE == T_Q5_K || TYPE == T_IQ3_S;
 
+// Q5_K: values less 16, and the 16 in the min term: d sc q - dmin mn = d sc (q - 16) + kappa, kappa = 16 d sc - dmin mn. Weights
+// without a mean times activations with one make d sc q and dmin mn cancel almost wholly, and what is rounded before they meet
+// shows; q - 16 and kappa are small by themselves. kappa and u = asc * bsum enter the matrix pipe as three bf16 parts each, 24
+// bits, what the int8 kernel of Q5_K's shorter products holds them in (per-256 scales: u = bsum, exact in two parts). Error of
+// 500 x 5376 -> 4624 on such rows 3.3e-7 (the int8 kernel 6.3e-7; q, mn and two parts of u 2.3e-5, with three 1.4e-6), on random
+// ones a third of the int8 kernel's. 2048 x 5120 -> 17408: 697 us against 683 of two parts and 806 of int8; 333 x 17408 -> 5120
+// 143.5, 146.5, 157 (the parts lie by superblock, 1 KB a load, where rows of them took a cache line each).
+template <int TYPE> constexpr bool kF16Centred = TYPE == T_Q5_K;
+
 // ---- prepass: the int8 activations as f16 in MFMA operand order, and (MINS) the mins operand u = asc * bsum split
 // into two bf16 parts (one 32-bit word per token and block: bf16 hi | lo << 16; per superblock the 8 words are the
-// bf16 MFMA's B operand, slot 8h + i = block 4h + i / 2, part i % 2).
+// bf16 MFMA's B operand, slot 8h + i = block 4h + i / 2, part i % 2). CENTRED: both parts of all tokens by superblock; PARTS = 3: u2
+// has the first and the third part the same way. asc null: u = bsum.
 // One thread per (token, 32-block, k-half h); consecutive threads take consecutive lanes of one operand piece
 // (token % 32, then h), so each wave writes whole 1 KB pieces. A thread writes lane (token % 32, h)'s 16 bytes of the
 // block's two pieces: chunk c = 0 holds elements 8h + perm8(i), chunk 1 elements 16 + 8h + perm8(i).
 // HALF: lane half h holds the 16 elements of half h (chunk c: 16h + 8c + perm8(i)) instead, for the types whose records keep
 // a half together (kF16Half).
-template <bool MINS, bool HALF>
+template <int PARTS, bool HALF, bool CENTRED>
 __global__ __launch_bounds__(256) void f16_act_kernel(const int8_t* aq, const float* asc, const int16_t* absum, int M,
-                                                      int M_stride, int ash, int Mp, int K, uint8_t* af, uint32_t* u) {
+                                                      int M_stride, int ash, int Mp, int K, uint8_t* af, uint32_t* u,
+                                                      uint32_t* u2) {
   const int nb = K / 32;
   const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
   const int lanei = (int)(gid & 63), h = lanei >> 5;
@@ -95,17 +107,21 @@ __global__ __launch_bounds__(256) void f16_act_kernel(const int8_t* aq, const fl
                   (2 * (b & 1)) * kF16Piece + lanei * 16;
   *(uint4*)(base) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
   *(uint4*)(base + kF16Piece) = make_uint4(hw[4], hw[5], hw[6], hw[7]);
-  if constexpr (MINS) {
+  if constexpr (PARTS > 0) {
     if (h == 0) {
       float uv = 0.0f;
       if (m < M) {
         const int bs = (int)absum[(size_t)(2 * b) * M_stride + m] + (int)absum[(size_t)(2 * b + 1) * M_stride + m];
-        uv = asc[(size_t)(b >> ash) * M_stride + m] * (float)bs;
+        uv = asc ? asc[(size_t)(b >> ash) * M_stride + m] * (float)bs : (float)bs;
       }
       const __bf16 uh = (__bf16)uv;
       const __bf16 ul = (__bf16)(uv - (float)uh);
-      u[(size_t)m * nb + b] =
+      const size_t at = CENTRED ? ((size_t)(b >> 3) * Mp + m) * 8 + (b & 7) : (size_t)m * nb + b;
+      u[at] =
           (uint32_t)__builtin_bit_cast(uint16_t, uh) | ((uint32_t)__builtin_bit_cast(uint16_t, ul) << 16);
+      if constexpr (PARTS == 3)
+        u2[at] = (uint32_t)__builtin_bit_cast(uint16_t, uh) |
+                 ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(uv - (float)uh - (float)ul)) << 16);
     }
   }
 }
@@ -116,8 +132,9 @@ struct F16Args {
   WView w;
   const uint8_t* af;   // prepass output
   const uint32_t* u;   // mins operand
+  const uint32_t* u2;  // (three parts: the first and third)
   const float* asc;
-  int M, M_stride;
+  int M, M_stride, Mp;  // (Mp: M rounded up to whole tiles)
   int ash;             // asc row of 32-block b: b >> ash (per-32 scales: 0; per-256: 3)
   float* C;
   int ldc, c_off, accumulate;
@@ -176,7 +193,8 @@ __device__ __forceinline__ F16Pay f16_load(const uint8_t* qrow, int blk, int h) 
 }
 
 // Block b (0..7) of a superblock with header hdr: the lane's 16 values times the integer block scale, as the two f16 operands
-template <int TYPE>
+// (CENTRED: values less 16)
+template <int TYPE, bool CENTRED>
 __device__ __forceinline__ void f16_decode(const F16Pay& p, uint4 hdr, int b, int h, const typename LdsFor<TYPE>::type* tab,
                                            f16x8& b0, f16x8& b1) {
   if constexpr (TYPE == T_Q4_K) {
@@ -185,8 +203,9 @@ __device__ __forceinline__ void f16_decode(const F16Pay& p, uint4 hdr, int b, in
     (void)mn;
     q4k_f16_decode(p.x, p.y, sc, 0x64006400u, b0, b1);
   } else {
-    // words w[k] of bytes u (elements 16h + 4k ..): (1024 + u) as f16 is 0x6400 | u, and (1024 + u) sc - (1024 + bias) sc is
-    // exact as in q4k_f16_decode (bias 128 takes IQ3_S's signed bytes, flipped to unsigned, back)
+    // words w[k] of bytes u (elements 16h + 4k ..): IQ3_S (1024 + u) as f16 is 0x6400 | u, and (1024 + u) sc - (1024 + bias) sc is
+    // exact as in q4k_f16_decode (bias 128 takes the signed bytes, flipped to unsigned, back). Q5_K u = 4 q under the exponent of
+    // 256, 0x5C00 | 4 q, where the offset less 16 fits too: (256 + q) sc - 272 sc, and 272 * 63 = 17136 is an f16 (1040 * 63 is not)
     uint32_t w[4];
     int sc;
     if constexpr (TYPE == T_Q5_K) {
@@ -194,10 +213,10 @@ __device__ __forceinline__ void f16_decode(const F16Pay& p, uint4 hdr, int b, in
       q4k_scale_min(hdr.y, hdr.z, hdr.w, b, sc, mn);
       (void)mn;
       const uint32_t hb = p.z >> (4 * h);
-      w[0] = (p.x & 0x0F0F0F0Fu) | ((hb & 0x01010101u) << 4);
-      w[1] = (p.y & 0x0F0F0F0Fu) | ((hb & 0x02020202u) << 3);
-      w[2] = ((p.x >> 4) & 0x0F0F0F0Fu) | ((hb & 0x04040404u) << 2);
-      w[3] = ((p.y >> 4) & 0x0F0F0F0Fu) | ((hb & 0x08080808u) << 1);
+      w[0] = ((p.x << 2) & 0x3C3C3C3Cu) | ((hb & 0x01010101u) << 6);
+      w[1] = ((p.y << 2) & 0x3C3C3C3Cu) | ((hb & 0x02020202u) << 5);
+      w[2] = ((p.x >> 2) & 0x3C3C3C3Cu) | ((hb & 0x04040404u) << 4);
+      w[3] = ((p.y >> 2) & 0x3C3C3C3Cu) | ((hb & 0x08080808u) << 3);
     } else {
       const uint32_t qh = ((b < 4 ? hdr.x : hdr.y) >> (8 * (b & 3) + 4 * h)) & 0xFu, sg = p.y >> (16 * h);
       sc = 1 + 2 * (int)((hdr.z >> (4 * b)) & 0xFu);
@@ -209,12 +228,13 @@ __device__ __forceinline__ void f16_decode(const F16Pay& p, uint4 hdr, int b, in
 #pragma unroll
       for (int k = 0; k < 4; ++k) w[k] ^= 0x80808080u;
     }
-    const _Float16 s = (_Float16)sc, o = (_Float16)(TYPE == T_IQ3_S ? -1152.0f : -1024.0f) * s;
+    constexpr uint32_t hi = TYPE == T_IQ3_S ? 0x64646464u : 0x5C5C5C5Cu;
+    const _Float16 s = (_Float16)sc, o = (_Float16)(TYPE == T_IQ3_S ? -1152.0f : CENTRED ? -272.0f : -256.0f) * s;
     const f16x2 sc2 = {s, s}, off2 = {o, o};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const f16x2 v0 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, w[k], 0x04020400u)) * sc2 + off2;
-      const f16x2 v1 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, w[k], 0x04030401u)) * sc2 + off2;
+      const f16x2 v0 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(hi, w[k], 0x04020400u)) * sc2 + off2;
+      const f16x2 v1 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(hi, w[k], 0x04030401u)) * sc2 + off2;
       f16x8& d = k < 2 ? b0 : b1;
       const int i = 4 * (k & 1);
       d[i] = v0[0];
@@ -223,6 +243,11 @@ __device__ __forceinline__ void f16_decode(const F16Pay& p, uint4 hdr, int b, in
       d[i + 3] = v1[1];
     }
   }
+}
+
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi});
 }
 
 // Work-group -> (128-row weight tile, 128-token tile, K piece); consecutive work-groups of one XCD (work-groups are dealt to
@@ -264,7 +289,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
   const int n_rows = a.w.rows;
   const int nbase = nt * kF16BN + wave * 32;
   const int nrow = min(nbase + lc, n_rows - 1);  // this lane's A-operand row
-  constexpr bool MINS = Traits<TYPE>::MINS;
+  constexpr bool CENTRED = kF16Centred<TYPE> && !DUMP, MINS = Traits<TYPE>::MINS && !CENTRED;
   static_assert(Traits<TYPE>::HB == 16, "16-byte headers");
   __shared__ typename LdsFor<TYPE>::type tab;
   lds_fill<TYPE>(&tab);
@@ -326,7 +351,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
       __builtin_amdgcn_sched_barrier(0);
       f16x8 aw[2][2];
 #pragma unroll
-      for (int bb = 0; bb < 2; ++bb) f16_decode<TYPE>(pay[bb], hdr, 2 * p + bb, h, &tab, aw[bb][0], aw[bb][1]);
+      for (int bb = 0; bb < 2; ++bb) f16_decode<TYPE, CENTRED>(pay[bb], hdr, 2 * p + bb, h, &tab, aw[bb][0], aw[bb][1]);
       const uint8_t* L = lds + cur * kF16PairBytes + lane * 16;
       if constexpr (S256) {
         // items block-major (k = 4 bb + t): consecutive MFMAs feed different token tiles' accumulators
@@ -425,6 +450,23 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
         dtab[wave][0][lc] = h2f(TYPE == T_IQ3_S ? hdr.w : hdr.x);
         if constexpr (MINS) dtab[wave][1][lc] = h2f(hdr.x >> 16);
       }
+      // kappa's parts for the blocks 4h + j: slots 2j, 2j + 1 hold parts (0, 0), (1, 1), (2, 0) (S256, with two parts of u: (2, 2))
+      u32x4_t kop[CENTRED ? 3 : 1];
+      if constexpr (CENTRED) {
+        const float d16 = 16.0f * h2f(hdr.x), dm = h2f(hdr.x >> 16);
+        const uint32_t m0 = 0x0F0F0F0Fu, m1 = 0x30303030u, m2 = 0x3F3F3F3Fu;
+        const uint32_t scw = h ? (hdr.w & m0) | ((hdr.y >> 2) & m1) : hdr.y & m2;
+        const uint32_t mnw = h ? ((hdr.w >> 4) & m0) | ((hdr.z >> 2) & m1) : hdr.z & m2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float k = fmaf(d16, (float)((scw >> (8 * j)) & 0xFFu), -dm * (float)((mnw >> (8 * j)) & 0xFFu));
+          kop[0][j] = bf16_pair(k, k);
+          const float r1 = k - __builtin_bit_cast(float, kop[0][j] & 0xFFFF0000u);
+          kop[1][j] = bf16_pair(r1, r1);
+          const float r2 = r1 - __builtin_bit_cast(float, kop[1][j] & 0xFFFF0000u);
+          kop[2][j] = bf16_pair(r2, S256 ? r2 : k);
+        }
+      }
       int mn[8];
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
@@ -450,6 +492,25 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
       }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
+        if constexpr (CENTRED) {
+          const size_t uo = ((size_t)s * a.Mp + m0 + 32 * t + lc) * 8 + 4 * h;
+          const bf16x8 u01 = __builtin_bit_cast(bf16x8, *(const uint4*)(a.u + uo));
+          f32x16 tk = zero16;
+          if constexpr (!S256) {
+            const bf16x8 u02 = __builtin_bit_cast(bf16x8, *(const uint4*)(a.u2 + uo));
+            tk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kop[2]), u02, tk, 0, 0, 0);
+          } else {
+            tk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kop[2]), u01, tk, 0, 0, 0);
+          }
+          tk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kop[1]), u01, tk, 0, 0, 0);
+          tk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kop[0]), u01, tk, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const float v = fmaf(dr[r], tq[t][r], tk[r]);
+            res[t][r] = S256 ? fmaf(sv256[t], v, res[t][r]) : v + res[t][r];
+          }
+          continue;
+        }
         if constexpr (!MINS) {
           const float sv = S256 ? sv256[t] : 1.0f;
 #pragma unroll
@@ -682,31 +743,35 @@ hipError_t f16_scratch(void** out, size_t* bytes, void** part) {
 
 template <int TYPE>
 static hipError_t go_f16(const GemmArgs& g, void* ws, hipStream_t s) {
-  constexpr bool MINS = Traits<TYPE>::MINS, HALF = kF16Half<TYPE>;
+  constexpr int PARTS = !Traits<TYPE>::MINS ? 0 : kF16Centred<TYPE> ? 3 : 2;
+  constexpr bool HALF = kF16Half<TYPE>, CENTRED = kF16Centred<TYPE>;
   const int M = g.M, K = g.w.K;
   const int Mp = (int)round_up((size_t)M, kF16BM);
   void* buf = ws;
   hipError_t e = hipSuccess;
   if (!buf) {
-    e = pool_alloc(&buf, f16_workspace_bytes(M, K), s);
+    e = pool_alloc(&buf, f16_workspace_bytes(TYPE, M, K), s);
     if (e != hipSuccess) return e;
   }
   uint8_t* af = (uint8_t*)buf;
   uint32_t* u = (uint32_t*)(af + round_up((size_t)Mp * K * 2, 256));
-  const size_t threads = (size_t)Mp * (K / 32) * 2;
+  uint32_t* u2 = u + (size_t)Mp * (K / 32);
+  const dim3 agrid((unsigned)(((size_t)Mp * (K / 32) * 2 + 255) / 256));
   // (the block-sum mode reads no activation scales: no mins operand)
   if (g.dbg_isum)
-    f16_act_kernel<false, HALF><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(g.aq, nullptr, nullptr, M,
-                                                                                       g.M_stride, 0, Mp, K, af, u);
+    f16_act_kernel<0, HALF, CENTRED><<<agrid, dim3(256), 0, s>>>(g.aq, nullptr, nullptr, M, g.M_stride, 0, Mp, K, af, u, u2);
+  else if (CENTRED && g.ash == 3)
+    f16_act_kernel<2, HALF, CENTRED><<<agrid, dim3(256), 0, s>>>(g.aq, nullptr, g.absum, M, g.M_stride, 0, Mp, K, af, u, u2);
   else
-    f16_act_kernel<MINS, HALF><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(g.aq, g.asc, g.absum, M,
-                                                                                      g.M_stride, g.ash, Mp, K, af, u);
+    f16_act_kernel<PARTS, HALF, CENTRED><<<agrid, dim3(256), 0, s>>>(g.aq, g.asc, g.absum, M, g.M_stride, g.ash, Mp, K, af, u, u2);
   e = hipGetLastError();
   if (e == hipSuccess) {
     F16Args a{};
     a.w = g.w;
     a.af = af;
+    a.Mp = Mp;
     a.u = u;
+    a.u2 = u2;
     a.asc = g.asc;
     a.M = M;
     a.M_stride = g.M_stride;

@@ -150,7 +150,7 @@ hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s);
 // Prompt GEMM on the f16 matrix pipe (qm_gemm_f16.hip): the types and shapes it takes, its per-call workspace, and
 // the launcher (ws = null: the workspace comes from a per-device stream-ordered pool). dbg_isum: block-sum mode.
 bool f16_gemm_supported(int type, int M, int rows, int K);
-size_t f16_workspace_bytes(int M, int K);
+size_t f16_workspace_bytes(int type, int M, int K);
 hipError_t launch_gemm_f16(int type, const GemmArgs& a, void* ws, hipStream_t s);
 // The current device's copies of the static scratch arrays for the allocation-free entry: ptr (bytes) the f16 path's
 // workspace, part (kSplitBytes) the partial tiles

@@ -158,7 +158,8 @@ int qmatmul_gemm(const qm_weight* w, const int8_t* aq, const float* asc, const i
  * with or without -DACT32): act32 = 1 is qmatmul_gemm; act32 = 0 reads per-256 activation scales (asc [K/256][M_stride],
  * K % 256 == 0) -- the same kernels, which then take the scale of 32-block b from row b / 8. The per-256 result
  * equals the reference's superblock form asc * (d * sum_b sc*isum - dmin * sum_b mn*bsum) (gemm.cl:413-447) up to
- * f32 rounding order. */
+ * f32 rounding order. (On the f16 pipe a superblock's integer block sums are added in f32: exactly below 2^24, which all but
+ * rows of the largest values and scales stay under, rounded to f32 beyond.) */
 int qmatmul_gemm_ex(const qm_weight* w, const int8_t* aq, const float* asc, const int16_t* absum, int M, int M_stride,
                     int act32, float* C, int ldc, int c_off, int accumulate, void* stream);
 
