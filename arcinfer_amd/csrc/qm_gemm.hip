@@ -1169,16 +1169,27 @@ static hipError_t dispatch_s16(int mode, const GemmArgs& a, hipStream_t s) {
   }
 }
 
-// A work-group alone on its CU: the int8 kernel's round takes half of a full one's time, the other two kernels' about 0.7 (IQ4_XS
-// 777 x 17408 -> 5120 357 us of 250 + 107, Q6_K 333 x 17408 -> 5120 301 of 400, Q4_K 1024 x 4096 -> 4096 71 of 101).
-// A call that takes a workspace costs the host about 28 us, 20 of them the pool's; the f16 path has one anyway.
+// The rates of the int8, per-16 and f16 kernels (gemm_split). int8: by the weight of the type's decode, Q8_0 2.95 to Q5_K 4.05;
+// zeroing C and adding the halves into it 6 us and 9 per 512 tiles of 64 x 128 results (less where they are partly empty), the
+// second kernel of cut tiles 9 us and 4: with that figure too low cut tiles lost to halves (IQ2_XXS 341 x 4096 -> 3776 41.4 us
+// against 36.6, IQ3_S 71 x 3072 -> 10896 37.9 against 32.8, Q8_0 384 x 12544 -> 4352 93 against 84). The other two kernels
+// never take halves; they are cut for a tenth or more.
 GemmSplit gemm_split_for(int type, int M, int rows, int K, bool f16) {
   if (!f16 && skinny_supported(type, true, M, rows, K)) return GemmSplit{0, 1, 0, false, 0.0f};
-  const int gx = (rows + 127) / 128, bm = f16 ? 128 : M <= 32 ? 32 : 64;
+  const int gx = (rows + 127) / 128, bm = f16 ? 128 : M <= 32 ? 32 : 64, tiles = gx * ((M + bm - 1) / bm);
+  const float fill = (float)M * (float)rows / ((float)tiles * (float)bm * 128.0f);
   const bool s16 = type == T_Q6_K || type == T_Q3_K || type == T_Q2_K || type == T_IQ1_M || type == T_IQ2_XS || type == T_IQ2_S;
-  const bool int8 = !f16 && !s16;
-  return gemm_split(gx * ((M + bm - 1) / bm), K / 256, bm, int8, int8 ? 0.5f : f16 ? 0.7f : 0.75f, int8 ? 4.2f : f16 ? 6.5f : 5.9f,
-                    f16 ? 0.0f : 28.0f);
+  if (f16) return gemm_split(tiles, K / 256, bm, fill, false, GemmRates{6.5f, 0.7f, 0.7f, 0, 0, 0, 0, 4.5f, 9.1f, 0, 0.1f, 0, 0, 0});
+  if (s16) return gemm_split(tiles, K / 256, bm, fill, false, GemmRates{5.9f, 0.75f, 0.75f, 0, 0, 0, 0, 4.1f, 4.1f, 28, 0.1f, 8, 0, 0});
+  const float us = type == T_Q8_0 || type == T_Q4_0 || type == T_Q2_0 ? 2.95f
+                   : type == T_Q5_K                                  ? 4.05f
+                   : type == T_Q4_K || type == T_IQ3_S               ? 3.65f
+                   : type == T_IQ1_S || type == T_IQ3_XXS            ? 3.45f
+                                                                     : 3.25f;
+  // (pieces of one tile lie on all XCDs, so every token tile reads the weight past their L2s: 4 TB/s, which the widest type meets)
+  const float stream = type == T_Q8_0 ? 1.0625f / 4.0e6f * (float)rows * (float)K * (float)(tiles / gx) : 0.0f;
+  return gemm_split(tiles, K / 256, bm, fill, true,
+                    GemmRates{us, 0.65f, 0.55f, 4, 1.8f, 5.8f, 9.1f, 9.3f, 4.4f, 24, 0.03f, 1, 0.5f, stream});
 }
 
 hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s) {

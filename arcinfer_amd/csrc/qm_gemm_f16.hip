@@ -570,17 +570,17 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_kernel(F16Args a) {
 
 // Q4_K: every prompt of 128 tokens and more. Q5_K and IQ3_S, whose int8 kernels run without a workspace: where the product
 // is long enough for the call to wait for the GPU (the workspace costs the host about 20 us), 128-token tiles waste at most a
-// fifth of their rows, and the tiles' time here, with the prepass's, is under the int8 kernel's by the two kernels' measured rates
-// (microseconds of a round's superblock: Q5_K 7.4 against 4.5 for half the tiles' size, IQ3_S 7.2 against 4.0; 2048 x 5120 -> 17408
-// Q5_K 771 -> 660 us, IQ3_S 695 -> 650; 512 x 5120 -> 5120 86.6 -> 72.7 and 79.3 -> 70.3; but 1024 x 4096 -> 4096, 256 tiles here
-// and 512 there, 86.7 against 79.7 and 84.7 against 71.9).
+// fifth of their rows, and the modelled time here, with the prepass's 7 us and 0.16 per million values, is under the int8 kernel's
+// (2048 x 5120 -> 17408 Q5_K 773 -> 697 us, IQ3_S 695 -> 650; 512 x 5120 -> 5120 86.6 -> 72.7 and 79.3 -> 70.3; but 1024 x 4096 ->
+// 4096, 256 tiles here and 512 there, 86.7 against 79.7 and 84.7 against 71.9, and Q5_K 1167 x 1792 -> 13120, 1030 tiles here, a
+// third round of six, 146 against 142).
 bool f16_gemm_supported(int type, int M, int rows, int K) {
   if (M < 128 || K % 256) return false;
   if (type == T_Q4_K) return true;
   if (type != T_Q5_K && type != T_IQ3_S) return false;
   if ((double)M * rows * K < 1.2e10 || round_up((size_t)M, kF16BM) * 4 > (size_t)M * 5) return false;
-  const float here = gemm_split_for(type, M, rows, K, true).cost * (type == T_Q5_K ? 7.4f : 7.2f) + (float)M * (float)K * 1e-6f;
-  return here < 0.97f * gemm_split_for(type, M, rows, K, false).cost * (type == T_Q5_K ? 4.5f : 4.0f);
+  const float here = 7.0f + 1.03f * gemm_split_for(type, M, rows, K, true).us + 0.16e-6f * (float)M * (float)K;
+  return here < gemm_split_for(type, M, rows, K, false).us;
 }
 
 // One memory pool per device for the per-call workspace (stream-ordered: concurrent calls on different streams get

@@ -89,41 +89,53 @@ struct GemmSplit {
   int from, splits;  // tiles [0, from) whole, [from, tiles) in `splits` pieces each (splits = 1: none)
   size_t bytes;      // partial tiles
   bool halves;       // uncut, two K halves added into a zeroed C
-  float cost;        // the call's time in superblocks of a full round
+  float us;          // the call's modelled time
 };
-// Rounds that n equal work-groups take; alone: the time of a round that fills half the slots or less (a work-group that has
-// its CU to itself runs faster than two that share it), as a part of a full one. Many rounds overlap and cost their share.
-inline float gemm_rounds(int n, float alone) {
-  const int rem = n % kGemmSlots;
-  if (n > 2 * kGemmSlots) return (float)n / kGemmSlots;
-  return (float)(n / kGemmSlots) + (rem == 0 ? 0.0f : 2 * rem <= kGemmSlots ? alone : 1.0f);
+// A kernel's times in microseconds, fitted to some 2000 measured products of 14 types (rms 3 %): `us` a superblock of a full round;
+// `alone`, `last` the part of it that a superblock of a round takes which fills half the slots or less (a work-group that has its
+// CU to itself runs faster than two that share it), as the only round or after another; what a call costs besides when it runs
+// whole (and per 512 work-groups), in halves (and per 512 of them, as far as they hold results) and cut (and per 512 pieces; `stream` at least);
+// `host` what a call with its own workspace takes the host (0: it has one anyway). A call is cut for a gain of `part` of its time
+// and of `least` us; `even`: how much of pieces that differ by a superblock runs as their mean (the rest as the longest).
+struct GemmRates {
+  float us, alone, last, whole, whole_wg, half, half_wg, cut, cut_wg, host, part, least, even, stream;
+};
+// Rounds that n equal work-groups take. (With more than two whole rounds the last one starts while others still run.)
+inline float gemm_rounds(int n, const GemmRates& g) {
+  const int f = n / kGemmSlots, rem = n % kGemmSlots;
+  if (rem == 0) return (float)f;
+  if (f >= 2) return (float)f + (2 * rem <= kGemmSlots ? 0.38f : 0.82f);
+  return (float)f + (2 * rem > kGemmSlots ? 1.0f : f ? g.last : g.alone);
 }
-// tiles of bm x 128 results, K of nsb superblocks; us: microseconds of a full round's superblock; host: those below which the
-// call would wait for its own workspace (0: it has one anyway); halves: a small product may add two K halves into a zeroed C.
-// A work-group costs its superblocks and about one more (its prologue and store). With more than one whole round the last one
-// starts while others still run, and cutting it measured level (Q4_K 2048 x 5120 -> 17408, 2176 tiles: 572 us either way), so
-// only products of fewer than 1024 tiles are cut, of K 2048 and more, for a tenth or more.
-inline GemmSplit gemm_split(int tiles, int nsb, int bm, bool halves, float alone, float us, float host) {
-  GemmSplit r{tiles, 1, 0, false, gemm_rounds(tiles, alone) * (float)(nsb + 1)};
+// tiles of bm x 128 results, filled to `fill`; K of nsb superblocks; halves: a small product may add two K halves into a zeroed C.
+// A work-group costs its superblocks and about one more (its prologue and store). With more than one whole round cutting the last
+// measured level (Q4_K 2048 x 5120 -> 17408, 2176 tiles: 572 us either way), so only products of fewer than 1024 tiles are
+// cut, of K 2048 and more.
+inline GemmSplit gemm_split(int tiles, int nsb, int bm, float fill, bool halves, const GemmRates& g) {
+  GemmSplit r{tiles, 1, 0, false, g.whole + g.whole_wg * (float)tiles / kGemmSlots + g.us * gemm_rounds(tiles, g) * (float)(nsb + 1)};
   const int full = tiles / kGemmSlots * kGemmSlots, rem = tiles - full;
   if (halves && nsb >= 8 && tiles < kGemmSlots) {
-    const float t = gemm_rounds(2 * tiles, alone) * (float)(nsb / 2 + 1) + 3.0f;  // (3: zeroing C, adding into it)
+    const float p = 2.0f * (float)tiles / kGemmSlots;
+    const float t = g.half + p * (g.half_wg * fill - 7.4f * (1.0f - fill)) + g.us * gemm_rounds(2 * tiles, g) * (0.5f * (float)nsb + 1.0f);
     // (up to one tile per CU always: IQ4_XS 333 x 17408 -> 5120, 240 tiles, 131 us in halves against 156, 200 x 5120 -> 5120, 160
-    //  tiles, 45 against 51; above, when the doubled grid does not take as many rounds)
-    if (2 * tiles <= kGemmSlots || t < r.cost) {
-      r.cost = t;
+    //  tiles, 45 against 51; above, unless whole tiles are faster: 416 tiles of Q5_K 777 x 4096 -> 4096
+    //  93 us in halves against 75, but 360 of IQ4_XS 142 x 3072 -> 15312, the last token tile nearly empty, 46.6 against 48.5)
+    if (2 * tiles <= kGemmSlots || 0.97f * t < r.us) {
+      r.us = t;
       r.halves = true;
     }
   }
   if (rem == 0 || full > kGemmSlots || nsb < 8) return r;
-  const float uncut = r.cost, whole = (float)(full / kGemmSlots) * (float)(nsb + 1);
-  for (int s = 2; s <= 8 && nsb / s >= 2; ++s) {
+  const float uncut = r.us, whole = (float)(full / kGemmSlots) * (float)(nsb + 1);
+  GemmRates pieces = g;
+  if (full) pieces.alone = g.last;
+  // (pieces of two superblocks only where there are few: IQ2_XXS 75 x 2560 -> 8800, 138 tiles in five, 28.6 us against 25.2 in halves)
+  for (int s = 2; s <= 8 && nsb / s >= (halves && rem > 128 ? 3 : 2); ++s) {
     const size_t bytes = (size_t)rem * s * bm * 128 * sizeof(float);
-    // (the second kernel about 0.7, the partial tiles' traffic 0.7 per 512 pieces of 64 x 128 results)
-    const float t = whole + gemm_rounds(rem * s, alone) * (float)((nsb + s - 1) / s + 1) + 0.7f +
-                    0.7f * (float)(rem * s) * (float)bm / (64.0f * 512.0f);
-    if (host > 0.0f && (uncut - fmaxf(t, host / us)) * us < 8.0f) continue;
-    if (t < r.cost && t < 0.9f * uncut && bytes <= kSplitBytes) r = GemmSplit{full, s, bytes, r.halves, t};
+    const float deep = g.even * (float)nsb / (float)s + (1.0f - g.even) * (float)((nsb + s - 1) / s) + 1.0f;  // a piece's superblocks
+    const float t = g.cut + g.cut_wg * (float)(rem * s) / kGemmSlots + g.us * (whole + gemm_rounds(rem * s, pieces) * deep);
+    const float least = fmaxf(t, fmaxf(g.host, g.stream * (float)rem / (float)tiles));
+    if (least < (1.0f - g.part) * uncut && least <= uncut - g.least && t < 0.999f * r.us && bytes <= kSplitBytes) r = GemmSplit{full, s, bytes, r.halves, t};
   }
   return r;
 }

@@ -1,0 +1,58 @@
+"""The dispatch rules of the dense products (host code of the built library, no GPU): at shapes where each side was measured, the
+call takes the faster one. Times in microseconds, whole call, one MI355X."""
+import ctypes
+
+import pytest
+
+from arcinfer_amd import formats as F
+from arcinfer_amd import qmatmul
+
+
+class Split(ctypes.Structure):
+    _fields_ = [("start", ctypes.c_int), ("splits", ctypes.c_int), ("bytes", ctypes.c_size_t), ("halves", ctypes.c_bool),
+                ("us", ctypes.c_float)]
+
+
+@pytest.fixture(scope="module")
+def rules():
+    lib = qmatmul.load_library()
+    split = lib._ZN2qm14gemm_split_forEiiiib
+    split.restype, split.argtypes = Split, [ctypes.c_int] * 4 + [ctypes.c_bool]
+    f16 = lib._ZN2qm18f16_gemm_supportedEiiii
+    f16.restype, f16.argtypes = ctypes.c_bool, [ctypes.c_int] * 4
+    return split, f16
+
+
+def deal(rules, qtype, M, N, K):
+    split, f16 = rules
+    use = f16(qtype, M, N, K)
+    s = split(qtype, M, N, K, use)
+    return ("f16 " if use else "") + ("cut %d" % s.splits if s.splits > 1 else "halves" if s.halves else "whole")
+
+
+@pytest.mark.parametrize("qtype,M,N,K,want", [
+    # cut tiles against K halves of the int8 kernel
+    (F.IQ2_XXS, 341, 3776, 4096, "halves"),   # 36.6 against 41.4 cut in four
+    (F.IQ2_XXS, 393, 3360, 3072, "halves"),   # 30.5, 36.4
+    (F.IQ3_S, 71, 10896, 3072, "halves"),     # 32.8, 37.9
+    (F.IQ1_S, 93, 8896, 2560, "halves"),      # 28.9, 33.0 in five
+    (F.IQ2_XXS, 74, 6896, 9216, "halves"),    # 48.9, 53.0 in two
+    (F.Q8_0, 384, 4352, 15616, "halves"),     # 101, 109 in five
+    (F.Q8_0, 384, 4352, 12544, "halves"),     # 84, 93
+    (F.Q8_0, 70, 5632, 10496, "cut 5") ,      # 46.2 in halves, 39.4
+    (F.Q4_K, 120, 5888, 13056, "cut 5"),      # 68.8 in halves, 55.4
+    (F.IQ4_XS, 339, 2048, 9472, "cut 5"),     # 50.1 in halves, 41.3
+    (F.IQ4_XS, 1115, 5584, 8704, "cut 3"),    # 792 tiles, whole 238, 216
+    # whole tiles against halves: more than one tile per CU
+    (F.IQ4_XS, 142, 15312, 3072, "halves"),   # 46.6 against 48.5 whole: a nearly empty token tile's halves cost little
+    (F.IQ3_S, 133, 14368, 3072, "halves"),    # 52.0, 54.1
+    (F.Q5_K, 777, 4096, 4096, "whole"),       # 93 in halves, 75
+    (F.Q8_0, 1005, 3328, 2304, "whole"),      # 52.8 in halves, 34.6
+    # the f16 kernel against int8
+    (F.Q5_K, 1167, 13120, 1792, "whole"),     # 142, 146 on f16: a third round of six tiles
+    (F.Q5_K, 333, 5120, 17408, "f16 cut 4"),  # 157 on int8, 143
+    (F.Q5_K, 2048, 17408, 5120, "f16 whole"), # 773, 697
+    (F.IQ3_S, 512, 5120, 5120, "f16 cut 3"),  # 78, 73
+])
+def test_prompt_products(rules, qtype, M, N, K, want):
+    assert deal(rules, qtype, M, N, K) == want
