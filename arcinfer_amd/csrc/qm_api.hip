@@ -658,7 +658,7 @@ int qmatmul_moe_grouped_ex(const qm_weight* gate, const qm_weight* up, const qm_
   // gate and up: one launch when they share a type the int8 kernel takes in one pass; otherwise the gate projection
   // into hf, then the up projection forming h from it
   const bool s16 = [](int t) { return t == QM_Q6_K || t == QM_IQ2_XS || t == QM_IQ2_S || t == QM_Q3_K; }(gate->type);
-  const bool few = gate->type == up->type && qm::moe_few(gate->type, L.slots, NE, Fv);
+  const bool few = gate->type == up->type && qm::moe_few(gate->type, L.slots, NE, E, Fv);
   const bool fused = gate->type == up->type && (!s16 || few);
   if (e == hipSuccess) {
     qm::GemmArgs a{};
@@ -704,7 +704,8 @@ int qmatmul_moe_grouped_ex(const qm_weight* gate, const qm_weight* up, const qm_
     a.slots = L.slots;
     a.max_tiles = L.max_tiles;
     a.expert_rows = E;
-    e = few ? qm::launch_moe_few(down->type, true, a, s) : qm::launch_gemm(down->type, qm::GEMM_MOE_DOWN, a, s);
+    e = qm::moe_few_down(down->type, L.slots, NE, E, F) ? qm::launch_moe_few(down->type, true, a, s)
+                                                        : qm::launch_gemm(down->type, qm::GEMM_MOE_DOWN, a, s);
   }
   if (e == hipSuccess) e = qm::launch_moe_combine(x, y, inv, T, NU, E, accumulate, shd, s);
   return e == hipSuccess ? QM_OK : hip_fail(e, "qmatmul_moe_grouped");

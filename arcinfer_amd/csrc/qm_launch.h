@@ -205,8 +205,9 @@ hipError_t launch_moe_scatter(const int* ids, const float* wts, int T, int NU, i
                               const int* counts, int* cursor, int* tstart, int* tiles, int tile_rows, int* stok,
                               float* swt, int* inv, hipStream_t s);
 // Expert products over the slot tiles for small expert sets (qm_moe_few.hip): gate and up of one type (hq / hsc), or down; and
-// whether a layer of `slots` slots, NE experts and expert width Fv takes them
-bool moe_few(int type, int slots, int NE, int Fv);
+// whether a layer of `slots` slots, NE experts, hidden E and expert width Fv (F padded) takes them
+bool moe_few(int type, int slots, int NE, int E, int Fv);
+bool moe_few_down(int type, int slots, int NE, int E, int F);
 hipError_t launch_moe_few(int type, bool down, const GemmArgs& a, hipStream_t s);
 hipError_t launch_moe_combine(float* x, const float* y, const int* inv, int T, int NU, int E, int accumulate,
                               const MoeShared& sh, hipStream_t s);

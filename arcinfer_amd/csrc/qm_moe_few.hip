@@ -238,14 +238,33 @@ static hipError_t few_go(bool down, const GemmArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// The prompt kernels launch about `wgs` work-groups for gate and up. Measured layers (IQ4_XS unless said, 2048 hidden, old -> new
-// us): 32 experts of 256, 96 slots (70 work-groups) 65 -> 41, 2048 slots (192) 89 -> 72; 32 of 768, 512 slots (288) 102 -> 80; 128 of
-// 256, 384 slots (280) 76 -> 60; Q6_K 32 of 256, 512 slots 129 -> 71; Q8_0, whose stream is twice as long, 32 of 768, 96 slots (210)
-// 86 -> 81 and 512 slots (288) 104 against 111. Level or slower beyond: 64 of 256, 2048 slots (256; 32 an expert) 100 against
-// 103, 256 of 512, 96 slots (396) 75 either way, 768 slots (1120) 167 against 201.
-bool moe_few(int type, int slots, int NE, int Fv) {
-  const int wgs = (Fv + 127) / 128 * ((slots < NE ? slots : NE) + slots / 32);
-  return wgs <= (type == T_Q8_0 ? 224 : 320) && (slots <= 16 * NE || wgs <= 192);
+// Which products come here: by the work-groups of 128 columns that the prompt kernels launch, wgs, and their decode (one pass, or two
+// for the types with scales per 16 elements, s16). The two are chosen apart, from 460 layers of 8 to 256 experts, E 768 to 4096, F 256
+// to 1024 and 66 to 6600 slots, each product on both (whole layers, us, old -> new); of those no layer is slower by over 3 %.
+// Gate and up: up to 256 (one a CU there; IQ4_XS 8 experts of 512, E 2048, 330 slots 91 -> 57, Q6_K 8 of 256, E 1792, 118 slots 107 ->
+// 48), 192 where an expert has many slots (IQ2_XXS 8 of 512, E 2048, 1812 slots, 256: 78 -> 87); to 320 where tiles are few, narrow or
+// nearly empty, or the prompt kernels run twice (but Q6_K 64 of 512, E 4096, 222 slots, 280: 155 -> 183). Q8_0, whose stream is
+// twice as long, to 128 (32 of 512, E 2048, 96 slots, 140: 67 -> 73), to 160 with over four slots an expert.
+static bool s16(int t) { return t == T_Q6_K || t == T_Q3_K || t == T_IQ2_XS || t == T_IQ2_S; }
+static int few_tiles(int slots, int NE) { return (slots < NE ? slots : NE) + slots / kMoeTileRows; }
+
+bool moe_few(int type, int slots, int NE, int E, int Fv) {
+  const int tiles = few_tiles(slots, NE), wgs = (Fv + 127) / 128 * tiles;
+  if (wgs > 192 && slots > 16 * NE) return false;
+  if (type == T_Q8_0) return wgs < 128 || (wgs <= 160 && slots > 4 * NE);
+  if (wgs <= 256 || wgs > 320) return wgs <= 256;
+  if (s16(type)) return type != T_Q6_K || E < 2048 || tiles <= 52 || slots <= 2 * NE;
+  return tiles <= 52 || Fv <= 256 || slots <= 4 * NE;
+}
+
+// Down, IQ4_XS 32 of 512, E 1024, 160 slots, 296: 66 -> 52; the prompt kernels catch up with more work-groups (E 4096, 1302 slots,
+// 2304: 137 -> 144) and longer rows (32 of 1024, E 2048, 220 slots, 608: Q8_0 90 -> 111; but 8 of 1024, E 1280, 164 slots, 130: IQ3_S
+// 72 -> 65).
+bool moe_few_down(int type, int slots, int NE, int E, int F) {
+  const int wgs = (E + 127) / 128 * few_tiles(slots, NE);
+  if (s16(type)) return wgs <= (slots > 16 * NE ? 256 : 200);
+  if (type == T_Q8_0) return wgs <= (F <= 512 ? 550 : F <= 768 ? 750 : 0);
+  return wgs <= 200 || (F <= 768 && (wgs <= 850 || (wgs <= (F > 512 ? 1600 : 1100) && slots <= 16 * NE)));
 }
 
 hipError_t launch_moe_few(int type, bool down, const GemmArgs& a, hipStream_t s) {

@@ -24,3 +24,15 @@ def test_slot_tile_edges(qm, dev, types, E, Fd):
     qm.moe_grouped(s["g"], s["u"], s["d"], NE, s["lgt"], NU, s["aq"], s["asc"], s["out"], s["ws"])
     torch.cuda.synchronize()
     moe_check(qm, s, types, NE, E, Fd, T, NU)
+
+
+@pytest.mark.parametrize("types,E,Fd", [
+    ((F.Q8_0, F.Q8_0, F.IQ4_XS), 256, 512),    # gate and up on the prompt kernels, down on the fine-grained one
+    ((F.IQ4_XS, F.IQ3_S, F.IQ2_XXS), 256, 256),  # gate and up of two types, one launch each
+    ((F.IQ4_XS, F.IQ4_XS, F.Q8_0), 512, 1024),  # the other way round
+])
+def test_one_product_of_the_two(qm, dev, types, E, Fd):
+    NE, NU, T = 32, 2, 35
+    s = _moe_setup(qm, dev, NE, E, Fd, T, NU, types[0], seed=5, types=types)
+    qm.moe_grouped(s["g"], s["u"], s["d"], NE, s["lgt"], NU, s["aq"], s["asc"], s["out"], s["ws"])
+    moe_check(qm, s, types, NE, E, Fd, T, NU)

@@ -1,4 +1,4 @@
-"""The dispatch rules of the dense products (host code of the built library, no GPU): at shapes where each side was measured, the
+"""The dispatch rules of the dense and expert products (host code of the built library, no GPU): at shapes where each side was measured, the
 call takes the faster one. Times in microseconds, whole call, one MI355X."""
 import ctypes
 
@@ -56,3 +56,39 @@ def deal(rules, qtype, M, N, K):
 ])
 def test_prompt_products(rules, qtype, M, N, K, want):
     assert deal(rules, qtype, M, N, K) == want
+
+
+@pytest.mark.parametrize("qtype,slots,NE,E,Fd,want", [
+    # gate and up on the fine-grained kernels (whole layer, prompt kernels' time against theirs)
+    (F.IQ4_XS, 330, 8, 2048, 512, True),    # 91, 57
+    (F.Q6_K, 118, 8, 1792, 256, True),      # 107, 48
+    (F.IQ4_XS, 268, 128, 2048, 256, True),  # 78, 59
+    (F.Q6_K, 222, 64, 4096, 512, False),    # 155, 183
+    (F.IQ2_XXS, 318, 64, 2048, 512, False), # 84, 86
+    (F.IQ2_XXS, 1812, 8, 2048, 512, False), # 78, 87
+    (F.IQ2_S, 72, 64, 2816, 512, True),     # 110, 71
+    (F.Q8_0, 96, 32, 2048, 512, False),     # 67, 73
+    (F.Q8_0, 108, 64, 2048, 512, False),    # 68, 81
+    (F.Q8_0, 198, 64, 4096, 256, False),    # 87, 93
+    (F.Q8_0, 660, 64, 1024, 256, False),    # 61, 63
+])
+def test_expert_gate_up(qtype, slots, NE, E, Fd, want):
+    few = qmatmul.load_library()._ZN2qm7moe_fewEiiiii
+    few.restype = ctypes.c_bool
+    assert few(qtype, slots, NE, E, Fd) == want
+
+
+@pytest.mark.parametrize("qtype,slots,NE,E,Fd,want", [
+    (F.IQ4_XS, 160, 32, 1024, 512, True),    # 66, 52
+    (F.IQ3_S, 164, 8, 1280, 1024, True),     # 72, 65
+    (F.IQ4_XS, 1302, 32, 4096, 512, False),  # 137, 144
+    (F.Q8_0, 220, 32, 2048, 1024, False),    # 90, 111
+    (F.Q8_0, 752, 128, 2048, 256, False),    # 98, 126
+    (F.Q8_0, 624, 64, 2048, 512, False),     # 90, 116
+    (F.Q6_K, 384, 64, 2048, 512, False),     # 94, 106
+    (F.Q6_K, 542, 32, 2048, 768, False),     # 140, 149
+])
+def test_expert_down(qtype, slots, NE, E, Fd, want):
+    few = qmatmul.load_library()._ZN2qm12moe_few_downEiiiii
+    few.restype = ctypes.c_bool
+    assert few(qtype, slots, NE, E, Fd) == want
