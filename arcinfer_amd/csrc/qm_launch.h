@@ -94,11 +94,11 @@ struct GemmSplit {
 // A kernel's times in microseconds, fitted to some 2000 measured products of 14 types (rms 3 %): `us` a superblock of a full round;
 // `alone`, `last` the part of it that a superblock of a round takes which fills half the slots or less (a work-group that has its
 // CU to itself runs faster than two that share it), as the only round or after another; what a call costs besides when it runs
-// whole (and per 512 work-groups), in halves (and per 512 of them, as far as they hold results) and cut (and per 512 pieces; `stream` at least);
+// whole (and per 512 work-groups), in halves (and per 512 of them, as far as they hold results, and as far as not) and cut (and per 512 pieces; `stream` at least);
 // `host` what a call with its own workspace takes the host (0: it has one anyway). A call is cut for a gain of `part` of its time
 // and of `least` us; `even`: how much of pieces that differ by a superblock runs as their mean (the rest as the longest).
 struct GemmRates {
-  float us, alone, last, whole, whole_wg, half, half_wg, cut, cut_wg, host, part, least, even, stream;
+  float us, alone, last, whole, whole_wg, half, half_wg, half_pad, cut, cut_wg, host, part, least, even, stream;
 };
 // Rounds that n equal work-groups take. (With more than two whole rounds the last one starts while others still run.)
 inline float gemm_rounds(int n, const GemmRates& g) {
@@ -116,7 +116,7 @@ inline GemmSplit gemm_split(int tiles, int nsb, int bm, float fill, bool halves,
   const int full = tiles / kGemmSlots * kGemmSlots, rem = tiles - full;
   if (halves && nsb >= 8 && tiles < kGemmSlots) {
     const float p = 2.0f * (float)tiles / kGemmSlots;
-    const float t = g.half + p * (g.half_wg * fill - 7.4f * (1.0f - fill)) + g.us * gemm_rounds(2 * tiles, g) * (0.5f * (float)nsb + 1.0f);
+    const float t = g.half + p * (g.half_wg * fill + g.half_pad * (1.0f - fill)) + g.us * gemm_rounds(2 * tiles, g) * (0.5f * (float)nsb + 1.0f);
     // (up to one tile per CU always: IQ4_XS 333 x 17408 -> 5120, 240 tiles, 131 us in halves against 156, 200 x 5120 -> 5120, 160
     //  tiles, 45 against 51; above, unless whole tiles are faster: 416 tiles of Q5_K 777 x 4096 -> 4096
     //  93 us in halves against 75, but 360 of IQ4_XS 142 x 3072 -> 15312, the last token tile nearly empty, 46.6 against 48.5)

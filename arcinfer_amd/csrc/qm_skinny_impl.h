@@ -433,9 +433,20 @@ static hipError_t skinny_route(const SkinnyArgs& a, hipStream_t s) {
 // Prompts: up to 16 tokens always (1.2-5.7 x); 17 to 32 unless the matrix is too large for one-tile work-groups to fit the
 // chip in a round or two and its rows too long for the sweep (17408 x 8192: IQ4_XS 54.5 against 63.0 us; Q6_K 89.6 against 84.7,
 // kept: its prompt kernel is slower).
+// Q8_0 prompts, whose int8 kernel decodes nothing: not from 24 tokens on at 4096 rows and more of over 2560 (31 x 4096 -> 4560 17.6 us
+// against 15.3), nor past 8192 rows of over 3072 where that kernel's K halves fill the chip once (20 x 3584 -> 15504 18.9 against 16.7,
+// 13 x 9216 -> 8304 34.8 against 27.6, 5 x 11264 -> 12640 43.1 against 32.8; but 9 x 7424 -> 22672, 178 column tiles, 35.8 against 41.9,
+// 9 x 4864 -> 10400, 82, 14.0 against 17.8).
+inline bool skinny_takes_q8(int M, int rows, int K) {
+  const int tiles = (rows + 127) / 128;
+  if (rows <= 8192) return M < 24 || rows <= 4096 || K <= 2560;
+  return K <= 3072 || (M <= 16 && (tiles > 128 || (K <= 5120 && tiles < 96)));
+}
+
 template <int TYPE>
 bool skinny_takes(bool prompt, int M, int rows, int K) {
   if (M > kSkinnyMax || M < 3) return prompt && M < 3;
+  if (prompt && TYPE == T_Q8_0) return skinny_takes_q8(M, rows, K);
   if (prompt) return M <= 16 || kHalves<TYPE> || rows <= 8192 || skinny_sweeps<TYPE>(M, rows, K);
   return M >= 5 || (K > 16384 && (M == 4 || K > 32768 || !kMin16<TYPE>)) || (Traits<TYPE>::QB == 16 && rows <= 8192 && K <= 5120);
 }

@@ -92,3 +92,24 @@ def test_expert_down(qtype, slots, NE, E, Fd, want):
     few = qmatmul.load_library()._ZN2qm12moe_few_downEiiiii
     few.restype = ctypes.c_bool
     assert few(qtype, slots, NE, E, Fd) == want
+
+
+@pytest.mark.parametrize("qtype,M,N,K,want", [
+    # prompts of up to 32 tokens on the few-token kernels (the prompt kernel's time against theirs)
+    (F.Q8_0, 12, 6016, 5376, True),     # 19.1, 11.2
+    (F.Q8_0, 30, 11376, 3072, True),    # 14.6, 11.9
+    (F.Q8_0, 9, 10400, 4864, True),     # 17.8, 14.0
+    (F.Q8_0, 9, 22672, 7424, True),     # 41.9, 35.8
+    (F.Q8_0, 28, 13296, 3584, False),   # 16.5, 19.3
+    (F.Q8_0, 20, 15504, 3584, False),   # 16.7, 18.9
+    (F.Q8_0, 4, 15600, 4608, False),    # 17.8, 19.7
+    (F.Q8_0, 9, 9792, 8192, False),     # 25.0, 33.8
+    (F.Q8_0, 5, 12640, 11264, False),   # 32.8, 43.1
+    (F.Q8_0, 31, 4560, 4096, False),    # 15.3, 17.6
+    (F.IQ4_XS, 13, 9952, 7168, True),
+    (F.Q6_K, 32, 17408, 17408, True),
+])
+def test_few_token_prompts(qtype, M, N, K, want):
+    takes = qmatmul.load_library()._ZN2qm16skinny_supportedEibiii
+    takes.restype, takes.argtypes = ctypes.c_bool, [ctypes.c_int, ctypes.c_bool] + [ctypes.c_int] * 3
+    assert takes(qtype, True, M, N, K) == want
