@@ -469,15 +469,14 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   } else {
     if (capturing) pb = 0;
     if (need + pb) {
-      e = qm::workspace_take(&call, need + pb, capturing, (hipStream_t)stream);
+      e = qm::workspace_take(&call, need, pb, capturing, (hipStream_t)stream);
       if (e == hipSuccess) {
         if (f16) scr = call.p;
-        if (pb) part = (float*)((uint8_t*)call.p + need);
+        if (pb && call.all) part = (float*)((uint8_t*)call.p + need);
       } else if (w->type == QM_Q4_K && f16) {
         return hip_fail(e, fn);
       } else {
         (void)hipGetLastError();  // (no memory: the int8 kernels, uncut, need none)
-        call.p = nullptr;
         f16 = false;
       }
     }

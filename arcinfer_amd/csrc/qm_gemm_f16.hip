@@ -583,134 +583,6 @@ bool f16_gemm_supported(int type, int M, int rows, int K) {
   return here < gemm_split_for(type, M, rows, K, false).us;
 }
 
-// One memory pool per device for the per-call workspace (stream-ordered: concurrent calls on different streams get
-// different buffers; the pool keeps freed memory for the next call).
-static hipError_t call_pool(hipMemPool_t* out) {
-  static std::mutex mu;
-  static hipMemPool_t pools[64] = {};
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
-  std::lock_guard<std::mutex> lock(mu);
-  if (!pools[dev]) {
-    hipMemPoolProps props{};
-    props.allocType = hipMemAllocationTypePinned;
-    props.location.type = hipMemLocationTypeDevice;
-    props.location.id = dev;
-    hipMemPool_t p;
-    e = hipMemPoolCreate(&p, &props);
-    if (e != hipSuccess) return e;
-    uint64_t thr = ~0ull;
-    e = hipMemPoolSetAttribute(p, hipMemPoolAttrReleaseThreshold, &thr);
-    if (e != hipSuccess) return e;
-    pools[dev] = p;
-  }
-  *out = pools[dev];
-  return hipSuccess;
-}
-
-hipError_t pool_alloc(void** out, size_t bytes, hipStream_t s) {
-  hipMemPool_t pool = nullptr;
-  const hipError_t e = call_pool(&pool);
-  return e == hipSuccess ? hipMallocFromPoolAsync(out, bytes, pool, s) : e;
-}
-
-// Kept workspaces. Taking a workspace from the pool and freeing it costs the host 10 to 30 us a call, and 50 to 70 us more
-// when other memory of the process was freed in between, which short prompts wait for. Up to 8 buffers a device
-// (32 MiB steps, 128 MiB at most each) stay allocated instead, one per stream that calls, as far as they go; each has an event
-// recorded behind its last use that the next user's stream waits for, so a buffer may move between streams and threads (a
-// stream's handle only says which buffer to prefer: handles are reused, the event is what orders). A buffer is out of the
-// list while a call enqueues its work. They are returned when the last weight is released.
-constexpr int kKeptMax = 8;
-constexpr size_t kKeptStep = (size_t)32 << 20, kKeptBytes = (size_t)128 << 20;
-struct KeptWs {
-  void* p = nullptr;
-  size_t bytes = 0;
-  hipEvent_t ev = nullptr;
-  hipStream_t last = nullptr;
-  bool busy = false;
-};
-static std::mutex g_kept_mu;
-static KeptWs g_kept[64][kKeptMax];
-
-hipError_t workspace_take(CallWs* ws, size_t bytes, bool capturing, hipStream_t s) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  *ws = CallWs{};
-  if (!capturing && dev >= 0 && dev < 64 && bytes <= kKeptBytes) {
-    std::lock_guard<std::mutex> lock(g_kept_mu);
-    int pick = -1, empty = -1;
-    for (int i = 0; i < kKeptMax; ++i) {
-      const KeptWs& k = g_kept[dev][i];
-      if (k.busy) continue;
-      if (!k.p) {
-        if (empty < 0) empty = i;
-      } else if (k.bytes >= bytes && (pick < 0 || (k.last == s && g_kept[dev][pick].last != s))) {
-        pick = i;
-      }
-    }
-    if ((pick < 0 || g_kept[dev][pick].last != s) && empty >= 0) {
-      KeptWs& k = g_kept[dev][empty];
-      const size_t size = round_up(bytes, kKeptStep);
-      e = k.ev ? hipSuccess : hipEventCreateWithFlags(&k.ev, hipEventDisableTiming);
-      if (e == hipSuccess) e = pool_alloc(&k.p, size, s);
-      if (e == hipSuccess) {
-        k.bytes = size;
-        k.last = s;
-        k.busy = true;
-        *ws = CallWs{k.p, empty};
-        return hipSuccess;
-      }
-      k.p = nullptr;
-      (void)hipGetLastError();
-    }
-    if (pick >= 0) {
-      KeptWs& k = g_kept[dev][pick];
-      e = hipStreamWaitEvent(s, k.ev, 0);
-      if (e == hipSuccess) {
-        k.last = s;
-        k.busy = true;
-        *ws = CallWs{k.p, pick};
-        return hipSuccess;
-      }
-      (void)hipGetLastError();
-    }
-  }
-  return pool_alloc(&ws->p, bytes, s);
-}
-
-hipError_t workspace_done(const CallWs& ws, hipStream_t s) {
-  if (ws.kept < 0) return hipFreeAsync(ws.p, s);
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;  // (the buffer stays out of the list)
-  e = hipEventRecord(g_kept[dev][ws.kept].ev, s);
-  if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lock(g_kept_mu);
-  g_kept[dev][ws.kept].busy = false;
-  return hipSuccess;
-}
-
-void workspaces_give_back() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
-  std::lock_guard<std::mutex> lock(g_kept_mu);
-  for (int d = 0; d < 64; ++d)
-    for (int i = 0; i < kKeptMax; ++i) {
-      KeptWs& k = g_kept[d][i];
-      if (!k.p || k.busy) continue;
-      if (hipSetDevice(d) != hipSuccess || hipEventSynchronize(k.ev) != hipSuccess || hipFreeAsync(k.p, nullptr) != hipSuccess) {
-        (void)hipGetLastError();
-        continue;
-      }
-      k.p = nullptr;
-      k.bytes = 0;
-    }
-  (void)hipSetDevice(dev);
-}
-
 // Allocation-free workspace for qmatmul_gemm_noalloc: a file-scope device array (each GPU holds its own copy until
 // the process ends). Host code never passes the array's name to a kernel or a copy -- in host code it is only a
 // stand-in for the symbol -- but the device address that hipGetSymbolAddress returns for the current device, looked

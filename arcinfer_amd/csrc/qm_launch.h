@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "qm_device.h"
+#include "qm_workspace.h"
 
 namespace qm {
 
@@ -144,19 +145,6 @@ GemmSplit gemm_split_for(int type, int M, int rows, int K, bool f16);
 // C (op)= the sums of the cut tiles' pieces (bm x 128 each); tile t: rows bm * (t % gy).., columns 128 * (t / gy).. when
 // m_fast, else bm * (t / gx).., 128 * (t % gx)..
 hipError_t launch_split_sum(const GemmArgs& a, int bm, int tiles, int gx, int gy, bool m_fast, hipStream_t s);
-// A per-device stream-ordered memory pool for per-call workspaces
-hipError_t pool_alloc(void** out, size_t bytes, hipStream_t s);
-// A per-call workspace of the current device, for work enqueued on s between the two calls: a buffer kept from an earlier call
-// (not on a capturing stream), ordered after that call's work, or memory of the pool. workspaces_give_back returns the kept
-// buffers of every device to their pools; no call may be enqueueing meanwhile.
-struct CallWs {
-  void* p = nullptr;
-  int kept = -1;  // index of the kept buffer, -1: the pool's
-};
-hipError_t workspace_take(CallWs* ws, size_t bytes, bool capturing, hipStream_t s);
-hipError_t workspace_done(const CallWs& ws, hipStream_t s);
-void workspaces_give_back();
-
 enum GemmMode : int { GEMM_DENSE = 0, GEMM_MOE_GATEUP = 1, GEMM_MOE_DOWN = 2, GEMM_MOE_G = 3, GEMM_MOE_UH = 4 };
 hipError_t launch_gemm(int type, int mode, const GemmArgs& a, hipStream_t s);
 // Prompt GEMM on the f16 matrix pipe (qm_gemm_f16.hip): the types and shapes it takes, its per-call workspace, and

@@ -1,0 +1,24 @@
+"""The prompt GEMM's per-call workspaces (csrc/qm_workspace.hip, host code): compiled against a HIP runtime on paper
+(fake_hip_workspace.cpp) whose memory and events are plain counters."""
+import os
+import subprocess
+
+import pytest
+
+from arcinfer_amd import build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROCM = os.path.dirname(os.path.dirname(build.HIPCC))
+
+
+@pytest.fixture(scope="module")
+def scenario(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("ws") / "ws")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"), "-I", build.CSRC, "-x", "c++",
+                    os.path.join(build.CSRC, "qm_workspace.hip"), os.path.join(HERE, "fake_hip_workspace.cpp"), "-o", exe], check=True)
+    return lambda name: [int(v) for v in subprocess.run([exe, name], check=True, capture_output=True, text=True).stdout.split()]
+
+
+def test_what_a_call_must_have_is_enough(scenario):
+    """24 MiB free, 20 needed, 30 more wanted: the call gets its 20 (without the rest) and leaves no error behind."""
+    assert scenario("need_alone") == [1, 0, 0]
