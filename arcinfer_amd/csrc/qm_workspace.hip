@@ -42,10 +42,10 @@ hipError_t pool_alloc(void** out, size_t bytes, hipStream_t s) {
 
 // Kept workspaces. Taking a workspace from the pool and freeing it costs the host 10 to 30 us a call, and 50 to 70 us more
 // when other memory of the process was freed in between, which short prompts wait for. Up to 8 buffers a device
-// (32 MiB steps, 128 MiB at most each) stay allocated instead, one per stream that calls, as far as they go; each has an event
-// recorded behind its last use that the next user's stream waits for, so a buffer may move between streams and threads (a
-// stream's handle only says which buffer to prefer: handles are reused, the event is what orders). A buffer is out of the
-// list while a call enqueues its work. They are returned when the last weight is released.
+// (32 MiB steps, 128 MiB at most each) stay allocated instead; each has an event recorded behind its last use. A call takes the one
+// that its stream used last (behind the event: a stream's handle only says which to prefer, handles are reused), or one whose work
+// has ended, or a new one, or else memory of the pool, so that no stream waits for another's work. A buffer is out of the list
+// while a call enqueues its work. They are returned when the last weight is released.
 constexpr int kKeptMax = 8;
 constexpr size_t kKeptStep = (size_t)32 << 20, kKeptBytes = (size_t)128 << 20;
 struct KeptWs {
@@ -55,6 +55,13 @@ struct KeptWs {
   hipStream_t last = nullptr;
   bool busy = false;
 };
+// whether the work of a buffer's last call has ended
+static bool ended(const KeptWs& k) {
+  if (hipEventQuery(k.ev) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 static std::mutex g_kept_mu;
 static KeptWs g_kept[64][kKeptMax];
 
@@ -63,7 +70,15 @@ static hipError_t take(CallWs* ws, size_t bytes, bool capturing, hipStream_t s) 
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   *ws = CallWs{};
+  // (a capture that the thread has open on another stream is none of this stream's business: its event queries and allocations
+  //  are no part of it, and must not end it)
+  struct Relaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  };
   if (!capturing && dev >= 0 && dev < 64 && bytes <= kKeptBytes) {
+    Relaxed relaxed;
     std::lock_guard<std::mutex> lock(g_kept_mu);
     int pick = -1, empty = -1;
     for (int i = 0; i < kKeptMax; ++i) {
@@ -71,11 +86,12 @@ static hipError_t take(CallWs* ws, size_t bytes, bool capturing, hipStream_t s) 
       if (k.busy) continue;
       if (!k.p) {
         if (empty < 0) empty = i;
-      } else if (k.bytes >= bytes && (pick < 0 || (k.last == s && g_kept[dev][pick].last != s))) {
+      } else if (k.bytes >= bytes && (k.last == s || (pick < 0 && ended(k)))) {
         pick = i;
+        if (k.last == s) break;
       }
     }
-    if ((pick < 0 || g_kept[dev][pick].last != s) && empty >= 0) {
+    if (pick < 0 && empty >= 0) {
       KeptWs& k = g_kept[dev][empty];
       const size_t size = (bytes + kKeptStep - 1) / kKeptStep * kKeptStep;
       e = k.ev ? hipSuccess : hipEventCreateWithFlags(&k.ev, hipEventDisableTiming);

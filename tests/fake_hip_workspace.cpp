@@ -80,6 +80,14 @@ int main(int argc, char** argv) {
     bool all = true;
     const bool ok = call(20 * MiB, 30 * MiB, 0, &all);
     printf("%d %d %d\n", ok, all, (int)last);
+  } else if (!strcmp(what, "streams")) {  // twelve streams with work in flight, twice; then one more stream, all work done
+    bool ok = true;
+    for (int turn = 0; turn < 2; ++turn)
+      for (int s = 0; s < 12; ++s) ok = ok && call(20 * MiB, 0, s);
+    const size_t kept = blocks.size(), calls = asked.size();
+    gpu_idle();
+    ok = ok && call(20 * MiB, 0, 99);
+    printf("%d %d %d %d %d\n", ok, waits - 8, (int)kept, (int)(asked.size() - calls), (int)last);  // (8: their own last calls)
   }
   return 0;
 }

@@ -22,3 +22,9 @@ def scenario(tmp_path_factory):
 def test_what_a_call_must_have_is_enough(scenario):
     """24 MiB free, 20 needed, 30 more wanted: the call gets its 20 (without the rest) and leaves no error behind."""
     assert scenario("need_alone") == [1, 0, 0]
+
+
+def test_no_stream_waits_for_another(scenario):
+    """Twelve streams, eight kept buffers: a stream waits for its own last call only, the other four have the pool's memory, and a
+    buffer whose work has ended serves any stream without a new allocation."""
+    assert scenario("streams") == [1, 0, 8, 0, 0]
