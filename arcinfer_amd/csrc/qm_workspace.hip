@@ -44,8 +44,8 @@ hipError_t pool_alloc(void** out, size_t bytes, hipStream_t s) {
 // when other memory of the process was freed in between, which short prompts wait for. Up to 8 buffers a device
 // (32 MiB steps, 128 MiB at most each) stay allocated instead; each has an event recorded behind its last use. A call takes the one
 // that its stream used last (behind the event: a stream's handle only says which to prefer, handles are reused), or one whose work
-// has ended, or a new one, or else memory of the pool, so that no stream waits for another's work. A buffer is out of the list
-// while a call enqueues its work. They are returned when the last weight is released.
+// has ended, or a new one in place of an empty slot or of a smaller buffer of these two kinds, or else memory of the pool, so
+// that no stream waits for another's work. A buffer is out of the list while a call enqueues its work. They are returned when the last weight is released.
 constexpr int kKeptMax = 8;
 constexpr size_t kKeptStep = (size_t)32 << 20, kKeptBytes = (size_t)128 << 20;
 struct KeptWs {
@@ -80,19 +80,30 @@ static hipError_t take(CallWs* ws, size_t bytes, bool capturing, hipStream_t s) 
   if (!capturing && dev >= 0 && dev < 64 && bytes <= kKeptBytes) {
     Relaxed relaxed;
     std::lock_guard<std::mutex> lock(g_kept_mu);
-    int pick = -1, empty = -1;
+    int pick = -1, place = -1;  // a buffer to take; the slot of a new one: the stream's own, an empty one, the smallest that has ended
     for (int i = 0; i < kKeptMax; ++i) {
       const KeptWs& k = g_kept[dev][i];
       if (k.busy) continue;
-      if (!k.p) {
-        if (empty < 0) empty = i;
-      } else if (k.bytes >= bytes && (k.last == s || (pick < 0 && ended(k)))) {
+      const bool own = k.p && k.last == s;
+      if (k.bytes >= bytes && (own || (pick < 0 && ended(k)))) {
         pick = i;
-        if (k.last == s) break;
+        if (own) break;
+      } else if (k.bytes < bytes) {
+        const KeptWs* q = place < 0 ? nullptr : &g_kept[dev][place];
+        if (!q || own || (!(q->p && q->last == s) && k.bytes < q->bytes))
+          if (own || !k.p || ended(k)) place = i;
       }
     }
-    if (pick < 0 && empty >= 0) {
-      KeptWs& k = g_kept[dev][empty];
+    if (pick < 0 && place >= 0) {
+      KeptWs& k = g_kept[dev][place];
+      if (k.p) {  // (freed behind the work of its last call)
+        if (hipStreamWaitEvent(s, k.ev, 0) != hipSuccess || hipFreeAsync(k.p, s) != hipSuccess) {
+          (void)hipGetLastError();
+          return pool_alloc(&ws->p, bytes, s);
+        }
+        k.p = nullptr;
+        k.bytes = 0;
+      }
       const size_t size = (bytes + kKeptStep - 1) / kKeptStep * kKeptStep;
       e = k.ev ? hipSuccess : hipEventCreateWithFlags(&k.ev, hipEventDisableTiming);
       if (e == hipSuccess) e = pool_alloc(&k.p, size, s);
@@ -100,7 +111,7 @@ static hipError_t take(CallWs* ws, size_t bytes, bool capturing, hipStream_t s) 
         k.bytes = size;
         k.last = s;
         k.busy = true;
-        *ws = CallWs{k.p, empty};
+        *ws = CallWs{k.p, place};
         return hipSuccess;
       }
       k.p = nullptr;

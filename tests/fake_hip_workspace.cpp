@@ -88,6 +88,17 @@ int main(int argc, char** argv) {
     gpu_idle();
     ok = ok && call(20 * MiB, 0, 99);
     printf("%d %d %d %d %d\n", ok, waits - 8, (int)kept, (int)(asked.size() - calls), (int)last);  // (8: their own last calls)
+  } else if (!strcmp(what, "grow")) {  // eight streams' small buffers, then one stream's larger call, three times; and a stream's own
+    bool ok = true;
+    for (int s = 0; s < 8; ++s) ok = ok && call(20 * MiB, 0, s);
+    gpu_idle();
+    size_t calls = asked.size();
+    for (int i = 0; i < 3; ++i) ok = ok && call(100 * MiB, 0, 99);
+    const int first = (int)(asked.size() - calls), kept = (int)blocks.size();
+    for (int s = 0; s < 8; ++s) ok = ok && call(20 * MiB, 0, s);  // (work in flight on every stream again)
+    calls = asked.size();
+    for (int i = 0; i < 3; ++i) ok = ok && call(50 * MiB, 0, 3);
+    printf("%d %d %d %d %d\n", ok, first, kept, (int)(asked.size() - calls), (int)blocks.size());
   }
   return 0;
 }

@@ -28,3 +28,8 @@ def test_no_stream_waits_for_another(scenario):
     """Twelve streams, eight kept buffers: a stream waits for its own last call only, the other four have the pool's memory, and a
     buffer whose work has ended serves any stream without a new allocation."""
     assert scenario("streams") == [1, 0, 8, 0, 0]
+
+
+def test_small_buffers_make_room(scenario):
+    """Eight small buffers don't send every larger call to the pool: it takes the place of one, once, and stays."""
+    assert scenario("grow") == [1, 1, 8, 1, 8]
