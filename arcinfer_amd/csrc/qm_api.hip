@@ -79,6 +79,16 @@ bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
 std::atomic<int> g_weights{0};  // prepared weights that are not released yet
 
+// hipMalloc, with the kept workspaces given back where memory is short
+hipError_t device_alloc(void** out, size_t bytes) {
+  hipError_t e = hipMalloc(out, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    if (qm::workspaces_give_back()) e = hipMalloc(out, bytes);
+  }
+  return e;
+}
+
 std::once_flag g_init_once;
 int g_init_status = QM_OK;
 char g_init_err[512] = "";
@@ -208,7 +218,7 @@ int qmatmul_prepare_weight(int type, const void* raw, int raw_on_device, int row
     delete w;
     return hip_fail(e, "qmatmul_prepare_weight: hipGetDevice");
   }
-  e = hipMalloc((void**)&w->base, total);
+  e = device_alloc((void**)&w->base, total);
   if (e != hipSuccess) {
     delete w;
     return fail(QM_ERR_NOMEM, "qmatmul_prepare_weight: hipMalloc(%zu): %s", total, hipGetErrorString(e));
@@ -216,7 +226,7 @@ int qmatmul_prepare_weight(int type, const void* raw, int raw_on_device, int row
   const uint8_t* src = (const uint8_t*)raw;
   uint8_t* staged = nullptr;
   if (!raw_on_device) {
-    e = hipMalloc((void**)&staged, rawb);
+    e = device_alloc((void**)&staged, rawb);
     if (e == hipSuccess) e = hipMemcpyAsync(staged, raw, rawb, hipMemcpyHostToDevice, s);
     if (e != hipSuccess) {
       if (staged) (void)hipFree(staged);
@@ -251,7 +261,7 @@ int qmatmul_release_weight(qm_weight* w) {
   if (!w) return fail(QM_ERR_ARG, "qmatmul_release_weight: null weight");
   hipError_t e = hipFree(w->base);
   delete w;
-  if (g_weights.fetch_sub(1) == 1) qm::workspaces_give_back();
+  if (g_weights.fetch_sub(1) == 1) (void)qm::workspaces_give_back();
   if (e != hipSuccess) return hip_fail(e, "qmatmul_release_weight: hipFree");
   return QM_OK;
 }

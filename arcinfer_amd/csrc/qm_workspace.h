@@ -9,7 +9,8 @@ namespace qm {
 hipError_t pool_alloc(void** out, size_t bytes, hipStream_t s);
 // A per-call workspace of the current device, for work enqueued on s between the two calls: a buffer kept from an earlier call
 // (not on a capturing stream), ordered after that call's work, or memory of the pool. `need` bytes, and `extra` behind them as far as
-// memory goes (all: they are there). workspaces_give_back returns the kept buffers that no call is using, of every device.
+// memory goes (all: they are there). workspaces_give_back waits for the kept buffers that no call is using, on every device, and
+// returns their memory to the device; false: there were none.
 struct CallWs {
   void* p = nullptr;
   int kept = -1;  // index of the kept buffer, -1: the pool's
@@ -17,6 +18,6 @@ struct CallWs {
 };
 hipError_t workspace_take(CallWs* ws, size_t need, size_t extra, bool capturing, hipStream_t s);
 hipError_t workspace_done(const CallWs& ws, hipStream_t s);
-void workspaces_give_back();
+bool workspaces_give_back();
 
 }  // namespace qm

@@ -62,6 +62,14 @@ static bool ended(const KeptWs& k) {
   return false;
 }
 
+// A capture that the thread has open on another stream is none of a call's business: event queries, allocations and frees made here
+// are no part of it and must not end it.
+struct Relaxed {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 static std::mutex g_kept_mu;
 static KeptWs g_kept[64][kKeptMax];
 
@@ -70,13 +78,6 @@ static hipError_t take(CallWs* ws, size_t bytes, bool capturing, hipStream_t s) 
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   *ws = CallWs{};
-  // (a capture that the thread has open on another stream is none of this stream's business: its event queries and allocations
-  //  are no part of it, and must not end it)
-  struct Relaxed {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-    ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-  };
   if (!capturing && dev >= 0 && dev < 64 && bytes <= kKeptBytes) {
     Relaxed relaxed;
     std::lock_guard<std::mutex> lock(g_kept_mu);
@@ -155,11 +156,14 @@ hipError_t workspace_done(const CallWs& ws, hipStream_t s) {
   return hipSuccess;
 }
 
-void workspaces_give_back() {
+bool workspaces_give_back() {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  bool any = false;
+  Relaxed relaxed;
   std::lock_guard<std::mutex> lock(g_kept_mu);
-  for (int d = 0; d < 64; ++d)
+  for (int d = 0; d < 64; ++d) {
+    bool here = false;
     for (int i = 0; i < kKeptMax; ++i) {
       KeptWs& k = g_kept[d][i];
       if (!k.p || k.busy) continue;
@@ -169,8 +173,16 @@ void workspaces_give_back() {
       }
       k.p = nullptr;
       k.bytes = 0;
+      here = true;
     }
+    // (a freed buffer stays the pool's, out of reach of any other allocation, until the pool is trimmed)
+    hipMemPool_t pool = nullptr;
+    if (here && (hipStreamSynchronize(nullptr) != hipSuccess || call_pool(&pool) != hipSuccess || hipMemPoolTrimTo(pool, 0) != hipSuccess))
+      (void)hipGetLastError();
+    any = any || here;
+  }
   (void)hipSetDevice(dev);
+  return any;
 }
 
 }  // namespace qm

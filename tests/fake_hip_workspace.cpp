@@ -99,6 +99,17 @@ int main(int argc, char** argv) {
     calls = asked.size();
     for (int i = 0; i < 3; ++i) ok = ok && call(50 * MiB, 0, 3);
     printf("%d %d %d %d %d\n", ok, first, kept, (int)(asked.size() - calls), (int)blocks.size());
+  } else if (!strcmp(what, "give_back")) {  // three streams' buffers, one of them in a call that is still enqueueing
+    bool ok = true;
+    for (int s = 0; s < 2; ++s) ok = ok && call(20 * MiB, 0, s);
+    qm::CallWs ws;
+    ok = ok && qm::workspace_take(&ws, 20 * MiB, 0, false, stream(2)) == hipSuccess;
+    qm::workspaces_give_back();
+    const int left = (int)blocks.size(), held = (int)(reserved / MiB);
+    ok = ok && qm::workspace_done(ws, stream(2)) == hipSuccess;
+    qm::workspaces_give_back();
+    ok = ok && call(20 * MiB, 0, 0);  // (and on as before)
+    printf("%d %d %d %d %d %d\n", ok, left, held, (int)blocks.size(), (int)(reserved / MiB), (int)last);
   }
   return 0;
 }

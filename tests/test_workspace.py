@@ -33,3 +33,8 @@ def test_no_stream_waits_for_another(scenario):
 def test_small_buffers_make_room(scenario):
     """Eight small buffers don't send every larger call to the pool: it takes the place of one, once, and stays."""
     assert scenario("grow") == [1, 1, 8, 1, 8]
+
+
+def test_given_back_to_the_device(scenario):
+    """What is given back leaves the pool too (32 MiB stay: the buffer of the call that is enqueueing), and the next call goes on."""
+    assert scenario("give_back") == [1, 1, 32, 1, 32, 0]
