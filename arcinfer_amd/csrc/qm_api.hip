@@ -410,6 +410,14 @@ int qmatmul_gemv_blocksums(const qm_weight* w, const int8_t* aq, const int16_t* 
   return e == hipSuccess ? QM_OK : hip_fail(e, "qmatmul_gemv_blocksums");
 }
 
+// whether a stream is (or may be: the query failed) under capture; a failed query leaves no error for the next launch's check
+static bool stream_captures(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // qmatmul_gemm, qmatmul_gemm_ex, qmatmul_gemm_ws and qmatmul_gemm_noalloc: one argument check and dispatch. act32 = 0
 // takes per-256 activation scales (asc [K/256][M_stride]); the kernels then read the scale of 32-block b at row b >> 3.
 // The workspace of the f16 path comes from the per-device pool (WS_POOL), the caller (WS_CALLER: ws, ws_bytes) or the
@@ -443,8 +451,7 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   a.ash = act32 ? 0 : 3;
   hipError_t e;
   const int K = w->view.K;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const bool capturing = wm == WS_POOL && (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone);
+  const bool capturing = stream_captures((hipStream_t)stream);
   void *scr = nullptr, *static_part = nullptr;
   size_t cap_bytes = 0;
   if (wm == WS_STATIC) {
