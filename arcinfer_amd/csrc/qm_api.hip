@@ -420,8 +420,8 @@ static bool stream_captures(hipStream_t s) {
 
 // qmatmul_gemm, qmatmul_gemm_ex, qmatmul_gemm_ws and qmatmul_gemm_noalloc: one argument check and dispatch. act32 = 0
 // takes per-256 activation scales (asc [K/256][M_stride]); the kernels then read the scale of 32-block b at row b >> 3.
-// The workspace of the f16 path comes from the per-device pool (WS_POOL), the caller (WS_CALLER: ws, ws_bytes) or the
-// static scratch array (WS_STATIC); every other case needs none.
+// Workspaces -- the f16 path's activations, which Q4_K must have, and the partial tiles of cut products, which no call must -- are
+// kept or pool memory (WS_POOL), the caller's (WS_CALLER: ws, ws_bytes) or the static arrays (WS_STATIC).
 enum WsMode { WS_POOL, WS_CALLER, WS_STATIC };
 
 static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const float* asc, const int16_t* absum,
@@ -454,16 +454,20 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
   const bool capturing = stream_captures((hipStream_t)stream);
   void *scr = nullptr, *static_part = nullptr;
   size_t cap_bytes = 0;
-  if (wm == WS_STATIC) {
-    e = qm::f16_scratch(&scr, &cap_bytes, &static_part);
-    if (e != hipSuccess) return hip_fail(e, "qmatmul_gemm_noalloc: scratch lookup");
-  }
-  // the f16 path's activations: Q4_K must have room for them; the other types of that path run on int8 MFMA without (and on a
-  // capturing stream, where they record no allocation)
+  // the f16 path's activations: Q4_K must have room for them; the other types of that path run on int8 MFMA without: on a capturing
+  // stream, where they record no allocation, and in the allocation-free entry, where they would share Q4_K's static array
   const size_t fb = qm::f16_workspace_bytes(w->type, M, K);
   bool f16 = qm::f16_gemm_supported(w->type, M, w->rows, K);
   if (f16 && w->type != QM_Q4_K)
-    f16 = wm == WS_STATIC ? fb <= cap_bytes : wm == WS_CALLER ? ws && ws_bytes >= fb && aligned(ws, 256) : !capturing;
+    f16 = wm == WS_CALLER ? ws && ws_bytes >= fb && aligned(ws, 256) : wm == WS_POOL && !capturing;
+  size_t need = f16 ? align256(fb) : 0;
+  qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, K, f16);
+  size_t pb = sp.splits > 1 ? sp.bytes : 0;  // partial tiles (optional)
+  if (capturing && wm != WS_CALLER) pb = 0;
+  if (wm == WS_STATIC && (f16 || pb)) {
+    e = qm::f16_scratch(&scr, &cap_bytes, &static_part);
+    if (e != hipSuccess) return hip_fail(e, "qmatmul_gemm_noalloc: scratch lookup");
+  }
   if (f16 && wm == WS_STATIC && fb > cap_bytes)
     return fail(QM_ERR_WORKSPACE, "%s: M %d x K %d needs %zu bytes of scratch, the static scratch holds %zu "
                 "(use qmatmul_gemm or qmatmul_gemm_ws)", fn, M, K, fb, cap_bytes);
@@ -474,28 +478,26 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
     if (!aligned(ws, 256)) return fail(QM_ERR_ARG, "%s: the workspace must be 256-byte aligned", fn);
     scr = ws;
   }
-  size_t need = f16 ? align256(fb) : 0;
-  qm::GemmSplit sp = qm::gemm_split_for(w->type, M, w->rows, K, f16);
-  size_t pb = sp.splits > 1 ? sp.bytes : 0;  // partial tiles (optional)
   qm::CallWs call;
   float* part = nullptr;
+  bool shared = false;
   if (wm == WS_STATIC) {
-    if (pb) part = (float*)static_part;
+    // (a call that may not use the array behind the last one runs uncut)
+    shared = pb && qm::shared_enter((hipStream_t)stream) == hipSuccess;
+    if (shared) part = (float*)static_part;
+    else (void)hipGetLastError();
   } else if (wm == WS_CALLER) {
     if (pb && ws && ws_bytes >= need + pb && aligned(ws, 256)) part = (float*)((uint8_t*)ws + need);
-  } else {
-    if (capturing) pb = 0;
-    if (need + pb) {
-      e = qm::workspace_take(&call, need, pb, capturing, (hipStream_t)stream);
-      if (e == hipSuccess) {
-        if (f16) scr = call.p;
-        if (pb && call.all) part = (float*)((uint8_t*)call.p + need);
-      } else if (w->type == QM_Q4_K && f16) {
-        return hip_fail(e, fn);
-      } else {
-        (void)hipGetLastError();  // (no memory: the int8 kernels, uncut, need none)
-        f16 = false;
-      }
+  } else if (need + pb) {
+    e = qm::workspace_take(&call, need, pb, capturing, (hipStream_t)stream);
+    if (e == hipSuccess) {
+      if (f16) scr = call.p;
+      if (pb && call.all) part = (float*)((uint8_t*)call.p + need);
+    } else if (w->type == QM_Q4_K && f16) {
+      return hip_fail(e, fn);
+    } else {
+      (void)hipGetLastError();  // (no memory: the int8 kernels, uncut, need none)
+      f16 = false;
     }
   }
   if (part) {
@@ -507,6 +509,10 @@ static int gemm_impl(const char* fn, const qm_weight* w, const int8_t* aq, const
           : qm::launch_gemm(w->type, qm::GEMM_DENSE, a, (hipStream_t)stream);
   if (call.p) {
     const hipError_t e2 = qm::workspace_done(call, (hipStream_t)stream);
+    if (e == hipSuccess) e = e2;
+  }
+  if (shared) {
+    const hipError_t e2 = qm::shared_leave((hipStream_t)stream);
     if (e == hipSuccess) e = e2;
   }
   return e == hipSuccess ? QM_OK : hip_fail(e, fn);

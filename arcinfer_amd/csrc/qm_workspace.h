@@ -20,4 +20,9 @@ hipError_t workspace_take(CallWs* ws, size_t need, size_t extra, bool capturing,
 hipError_t workspace_done(const CallWs& ws, hipStream_t s);
 bool workspaces_give_back();
 
+// Use of the current device's static partial-tile array by work enqueued on s between enter and leave: behind the work of the call
+// that used it before, on whatever stream, and other threads' calls wait outside. Not on a capturing stream.
+hipError_t shared_enter(hipStream_t s);
+hipError_t shared_leave(hipStream_t s);
+
 }  // namespace qm

@@ -185,4 +185,32 @@ bool workspaces_give_back() {
   return any;
 }
 
+struct Shared {
+  std::mutex mu;
+  hipEvent_t ev = nullptr;
+};
+static Shared g_shared[64];
+
+hipError_t shared_enter(hipStream_t s) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+  Shared& g = g_shared[dev];
+  Relaxed relaxed;
+  g.mu.lock();
+  e = g.ev ? hipStreamWaitEvent(s, g.ev, 0) : hipEventCreateWithFlags(&g.ev, hipEventDisableTiming);
+  if (e != hipSuccess) g.mu.unlock();
+  return e;
+}
+
+hipError_t shared_leave(hipStream_t s) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  e = hipEventRecord(g_shared[dev].ev, s);
+  g_shared[dev].mu.unlock();
+  return e;
+}
+
 }  // namespace qm

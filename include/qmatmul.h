@@ -148,7 +148,8 @@ int qmatmul_gemv(const qm_weight* w, const int8_t* aq, const float* asc, const i
  * Q5_K and IQ3_S, run on the f16 matrix pipe (exact integer block sums from f16 products) with a per-call workspace of about
  * 2*M*K bytes; products of few tiles, or of few more than the chip holds at once, are cut along K and take up to 32 MiB for the
  * pieces' partial results; every other case runs on int8 MFMA without. The workspace is one of a few buffers kept between
- * calls (at most 8 of 128 MiB a device, returned when the last weight is released; calls on any streams and threads may
+ * calls (at most 8 of 128 MiB a device, returned when the last weight is released and when a weight's preparation finds no memory;
+ * calls on any streams and threads may
  * overlap) or memory of a per-device stream-ordered pool. On a stream under capture only Q4_K takes one (the pool's); the others
  * then run uncut on int8 MFMA, equal up to f32 rounding order, as they do when there is no memory. A caller
  * that owns all memory passes the workspace itself (qmatmul_gemm_ws). */
@@ -175,14 +176,14 @@ int qmatmul_gemm_ws(const qm_weight* w, const int8_t* aq, const float* asc, cons
 
 /* qmatmul_gemm without any device allocation. No counterpart in the reference: for callers that cannot allocate
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc). Same arguments, results and kernels
- * as qmatmul_gemm; where qmatmul_gemm would take its pool workspace, this entry uses two static 32 MiB device arrays
- * (on each GPU, held until the process ends), one for the f16 path, one for partial results, and returns
- * QM_ERR_WORKSPACE when the f16 path needs more
- * (2*Mp*K + 4*Mp*K/32 bytes, Mp = M rounded up to 128; e.g. M 2048 x K 5120 needs 22.3 MB).
- * Every call on one GPU shares that GPU's arrays: calls that overlap on one GPU (different streams, or threads) race
- * and must be ordered by the caller. Each call writes every scratch byte it reads before reading it. It takes per-32
- * activation scales only (qmatmul_gemm's act32 = 1); a caller with per-256 scales that cannot allocate passes its
- * own workspace to qmatmul_gemm_ws. */
+ * as qmatmul_gemm, but that Q5_K and IQ3_S run on int8 MFMA alone (equal up to f32 rounding order). Where qmatmul_gemm would take a
+ * workspace, this entry uses two static 32 MiB device arrays (on each GPU, held until the process ends): one for the f16 path of
+ * Q4_K with M >= 128, which returns QM_ERR_WORKSPACE when it needs more (2*Mp*K + 4*Mp*K/32 bytes, Mp = M rounded up to 128; e.g.
+ * M 2048 x K 5120 needs 22.3 MB), and one for the partial results of cut products, whose calls are ordered one behind the other on
+ * the GPU; on a stream under capture no product is cut. Q4_K calls with M >= 128 that overlap on one GPU (different streams, or
+ * threads) race and must be ordered by the caller; all others may overlap. Each call writes every scratch byte it reads before
+ * reading it. It takes per-32 activation scales only (qmatmul_gemm's act32 = 1); a caller with per-256 scales that cannot allocate
+ * passes its own workspace to qmatmul_gemm_ws. */
 int qmatmul_gemm_noalloc(const qm_weight* w, const int8_t* aq, const float* asc, const int16_t* absum, int M,
                          int M_stride, float* C, int ldc, int c_off, int accumulate, void* stream);
 

@@ -110,6 +110,13 @@ int main(int argc, char** argv) {
     qm::workspaces_give_back();
     ok = ok && call(20 * MiB, 0, 0);  // (and on as before)
     printf("%d %d %d %d %d %d\n", ok, left, held, (int)blocks.size(), (int)(reserved / MiB), (int)last);
+  } else if (!strcmp(what, "shared")) {  // two streams' use of the one array, in turn
+    bool ok = true;
+    for (int i = 0; i < 4; ++i) {
+      ok = ok && qm::shared_enter(stream(i & 1)) == hipSuccess;
+      ok = ok && qm::shared_leave(stream(i & 1)) == hipSuccess;
+    }
+    printf("%d %d\n", ok, waits);
   }
   return 0;
 }

@@ -38,3 +38,8 @@ def test_small_buffers_make_room(scenario):
 def test_given_back_to_the_device(scenario):
     """What is given back leaves the pool too (32 MiB stay: the buffer of the call that is enqueueing), and the next call goes on."""
     assert scenario("give_back") == [1, 1, 32, 1, 32, 0]
+
+
+def test_shared_array_is_used_in_turn(scenario):
+    """Four uses from two streams: each but the first waits on the GPU for the one before."""
+    assert scenario("shared") == [1, 3]

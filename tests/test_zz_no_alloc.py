@@ -55,3 +55,55 @@ def test_noalloc_int8_path_and_capacity(qm, dev):
     torch.cuda.synchronize()
     assert bool(torch.all(C == 3.0))
     w.release()
+
+
+def test_noalloc_calls_overlap(qm, dev):
+    """Cut products (IQ4_XS, Q6_K) of two streams in turn without a wait between: each the result of the call by itself, and of
+    qmatmul_gemm, though their partial results share one array; and two captured ones replayed together."""
+    import torch
+    M, K = 70, 8192
+    cases = [_case(qm, dev, F.IQ4_XS, M, 272, K, 11), _case(qm, dev, F.Q6_K, M, 400, K, 13)]
+    want = [qm.gemm(*c, M=M) for c in cases]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    out = [[torch.empty_like(w) for _ in range(20)] for w in want]
+    torch.cuda.synchronize()
+    for i in range(20):
+        for c, o, s in zip(cases, out, streams):
+            qm.gemm(*c, M=M, C=o[i], ldc=c[0].rows, noalloc=True, stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    assert all(torch.equal(C, w) for o, w in zip(out, want) for C in o)
+    uncut = [qm.gemm_ws(*c, None, M=M) for c in cases]
+    graphs = [torch.cuda.CUDAGraph() for _ in cases]
+    for g, c, o in zip(graphs, cases, out):
+        with torch.cuda.graph(g):
+            qm.gemm(*c, M=M, C=o[0], ldc=c[0].rows, noalloc=True)
+    for _ in range(3):
+        for o in out:
+            o[0].zero_()
+        torch.cuda.synchronize()
+        for g, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o[0], u) for o, u in zip(out, uncut))
+    for c in cases:
+        c[0].release()
+
+
+def test_gemm_beside_a_capture(qm, dev):
+    """A call on one stream while the thread has a capture open on another: neither disturbs the other."""
+    import torch
+    w, aq, asc, absum = _case(qm, dev, F.IQ4_XS, 70, 272, 8192, 17)
+    want, uncut = qm.gemm(w, aq, asc, absum, M=70), qm.gemm_ws(w, aq, asc, absum, None, M=70)
+    side, C, D = torch.cuda.Stream(), torch.zeros_like(want), torch.zeros_like(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        qm.gemm(w, aq, asc, absum, M=70, C=C, ldc=272)
+        qm.gemm(w, aq, asc, absum, M=70, C=D, ldc=272, stream=side.cuda_stream)
+    for _ in range(2):
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, uncut) and torch.equal(D, want)
+    w.release()
