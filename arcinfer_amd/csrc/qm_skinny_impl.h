@@ -140,13 +140,19 @@ __device__ __forceinline__ void quad_product(const SkinnyArgs& a, const RawBlk& 
         sk_v4i s[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) s[j] = sums(h, j);
+        // (one token tile: the second half's sum by itself, as one chain of eight rounds more than two of four)
+        constexpr bool APART = NT == 1;
+        sk_v4f hs = sum;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float v = (float)s[j][r];
-            sum[r] = !Traits<TYPE>::MINS && h == 0 && j == 0 ? scl[r] * v : fmaf(scl[4 * j + r], v, sum[r]);
+            const bool first = j == 0 && (h == 0 ? !Traits<TYPE>::MINS : APART);
+            hs[r] = first ? scl[r] * v : fmaf(scl[4 * j + r], v, hs[r]);
           }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] = h > 0 && APART ? sum[r] + hs[r] : hs[r];
         // (one half and token tile at a time: free to move, the compiler starts them all and runs out of registers)
         if constexpr (HALVES) __builtin_amdgcn_sched_barrier(0);
       }
@@ -156,15 +162,16 @@ __device__ __forceinline__ void quad_product(const SkinnyArgs& a, const RawBlk& 
   }
 }
 
-// Adds the W waves' partial tiles (part[wave][element][lane], element = 4 * tile + r) in wave order and stores NTOT result
+// Adds the W waves' partial tiles (part[wave][element][lane], element = 4 * tile + r) in 64 bits and stores NTOT result
 // tiles; tile e / 4 is token tile (e / 4) % NT of row tile (e / 4) / NT from row n0.
 template <int NT, int NTOT, int W>
 __device__ __forceinline__ void store_tiles(const SkinnyArgs& a, const float (*part)[NTOT * 4][64], int n0, int wave) {
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   for (int e = wave; e < NTOT * 4; e += W) {
-    float v = part[0][e][lane];
+    double sum = part[0][e][lane];
 #pragma unroll
-    for (int k = 1; k < W; ++k) v += part[k][e][lane];
+    for (int k = 1; k < W; ++k) sum += (double)part[k][e][lane];
+    float v = (float)sum;
     const int t = 16 * ((e >> 2) % NT) + 4 * g + (e & 3), n = n0 + 16 * ((e >> 2) / NT) + c;
     if (t < a.M && n < a.w.rows) {
       float* cp = a.C + (size_t)t * a.ldc + a.c_off + n;
@@ -180,7 +187,9 @@ __device__ __forceinline__ void store_tiles(const SkinnyArgs& a, const float (*p
 }
 
 // A work-group owns RT row tiles; its W waves split K (wave w: quads w, w + W, ...), each with PF quads' loads in flight.
-// Tokens are read from L2 with every quad (two row tiles halve that), so any K goes.
+// Tokens are read from L2 with every quad (two row tiles halve that), so any K goes. Every fourth quad a wave's one tile
+// (decode) goes to 64 bits: added up in f32, 34 quads a wave, 5 tokens of 17408 were 1.27e-7 off the exact product against the GEMV's 8.8e-8; now 7.2e-8, for 1
+// to 4 % of the time (every eighth quad: as long, and up to 1.07 of the GEMV's error).
 template <int TYPE, int RT, int NT, int W, int PF, bool DUMP>
 __global__ __launch_bounds__(64 * W, 4) void skinny_kernel(SkinnyArgs a) {
   using Tr = Traits<TYPE>;
@@ -243,6 +252,16 @@ __global__ __launch_bounds__(64 * W, 4) void skinny_kernel(SkinnyArgs a) {
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = sk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  constexpr bool WIDE = !DUMP && RT * NT == 1;  // (decode's one tile; more have no registers for it)
+  double tot[WIDE ? 4 : 1] = {};
+  auto fold = [&] {
+    if constexpr (WIDE)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        tot[r] += (double)acc[0][0][r];
+        acc[0][0][r] = 0.0f;
+      }
+  };
   auto step = [&](int i, const Stage& s) {
     TokQuad<TYPE> tk[NT];
 #pragma unroll
@@ -263,17 +282,20 @@ __global__ __launch_bounds__(64 * W, 4) void skinny_kernel(SkinnyArgs a) {
       fetch(i + p + PF, st[p]);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (WIDE)
+      if (i & PF) fold();
   }
 #pragma unroll
   for (int p = 0; p < PF - 1; ++p)
     if (i + p < steps) step(i + p, st[p]);
   if constexpr (!DUMP) {
+    fold();
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) part[wave][(rt * NT + nt) * 4 + r][lane] = acc[rt][nt][r];
+        for (int r = 0; r < 4; ++r) part[wave][(rt * NT + nt) * 4 + r][lane] = WIDE ? (float)tot[WIDE ? r : 0] : acc[rt][nt][r];
     __syncthreads();
     store_tiles<NT, RT * NT, W>(a, part, n0, wave);
   }
