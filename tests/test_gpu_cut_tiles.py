@@ -11,9 +11,18 @@ from .test_gpu_parity import TOL_INT8_PATH, acts, assert_elementwise, rel_err, t
 pytestmark = pytest.mark.gpu
 
 # (type, M, N, K): the f16, int8 and per-16 kernels; partial row and column tiles; superblocks that do not divide evenly over
-# the pieces; 522 tiles, of which the last ten are cut
+# the pieces; 522 tiles, of which the last ten are cut, and 520 of the f16 kernel's (128 x 128), of which the last eight are
 CASES = [(F.Q4_K, 130, 144, 2048), (F.Q4_K, 300, 272, 5888), (F.IQ4_XS, 70, 272, 8192), (F.IQ3_S, 64, 144, 17408),
-         (F.Q6_K, 70, 272, 2304), (F.Q2_K, 129, 144, 4096), (F.IQ4_XS, 520, 7376, 4096), (F.Q6_K, 520, 7376, 2816)]
+         (F.Q6_K, 70, 272, 2304), (F.Q2_K, 129, 144, 4096), (F.IQ4_XS, 520, 7376, 4096), (F.Q6_K, 520, 7376, 2816),
+         (F.Q4_K, 600, 13232, 2304)]
+
+
+def f16_bytes(qtype, M, K):
+    """Workspace of the f16 kernel's activations alone, to whole 256 bytes (0 for the types and sizes of the other kernels)."""
+    if qtype not in (F.Q4_K, F.Q5_K, F.IQ3_S) or M < 128:
+        return 0
+    Mp = (M + 127) // 128 * 128
+    return (2 * Mp * K + Mp * (K // 32) * (8 if qtype == F.Q5_K else 4) + 255) // 256 * 256
 
 
 @pytest.mark.parametrize("qtype,M,N,K", CASES)
@@ -23,7 +32,7 @@ def test_cut_tiles(qm, dev, qtype, M, N, K):
     aq, asc, absum = acts(qm, F.synth_activations(M, K, seed=K, outlier_frac=0.01), dev, M_stride=M + 3)
     w = qm.QWeight(qtype, to_dev(W, dev), N, K)
     need = qm.gemm_workspace_size(w, M)
-    assert need > (2 * M * K if qtype == F.Q4_K else 0)  # (room for partial tiles: the call is cut)
+    assert need > f16_bytes(qtype, M, K)  # (room for partial tiles: the call is cut)
     C = qm.gemm(w, aq, asc, absum, M=M)
     ws = torch.empty((need,), dtype=torch.uint8, device=dev)
     assert torch.equal(C, qm.gemm_ws(w, aq, asc, absum, ws, M=M))
@@ -80,16 +89,18 @@ def test_captured_call_matches(qm, dev):
 
 @pytest.mark.parametrize("qtype", [F.Q5_K, F.IQ3_S])
 @pytest.mark.parametrize("act32", [True, False])
-def test_f16_types(qm, dev, qtype, act32):
-    """Q5_K and IQ3_S products long enough for the f16 kernels (ragged rows and tokens, whole and cut tiles): f32 parity, block
+@pytest.mark.parametrize("shape", [(500, 4624, 5376), (600, 13232, 3072)])
+def test_f16_types(qm, dev, qtype, act32, shape):
+    """Q5_K and IQ3_S products long enough for the f16 kernels (ragged rows and tokens; all tiles cut, and 512 whole with the last
+    eight cut): f32 parity, block
     sums bit for bit, and the int8 kernels behind the same call without a workspace."""
     import torch
-    M, N, K = 500, 4624, 5376
+    M, N, K = shape
     W = F.synth_weight(qtype, N, K, seed=qtype)
     x = F.synth_activations(M, K, seed=K, outlier_frac=0.01)
     aq, asc, absum = qm.quantize_act(to_dev(x, dev), M_stride=M + 3, act32=act32)
     w = qm.QWeight(qtype, to_dev(W, dev), N, K)
-    assert qm.gemm_workspace_size(w, M) > 2 * M * K
+    assert qm.gemm_workspace_size(w, M) > f16_bytes(qtype, M, K)  # (the f16 kernel, and cut)
     C = qm.gemm(w, aq, asc, absum, M=M, act32=act32)
     D = qm.gemm_ws(w, aq, asc, absum, None, M=M, act32=act32)
     torch.cuda.synchronize()
@@ -148,19 +159,31 @@ def test_kept_workspaces_over_streams_and_threads(qm, dev):
 
 
 @pytest.mark.parametrize("qtype", [F.IQ4_XS, F.IQ4_NL])
-def test_four_row_tiles(qm, dev, qtype):
+@pytest.mark.parametrize("K,act32", [(256, True), (768, True), (1280, False)])
+def test_four_row_tiles(qm, dev, qtype, K, act32):
     """Products of 1280 tiles of 128 x 128 and more (four row tiles per work-group for these types), the last row and column
-    tile ragged: parity on sampled columns, block sums bit for bit on the first and last rows."""
+    tile ragged, one superblock and odd numbers of them: parity on sampled columns, every accumulate mode, and block sums bit for
+    bit on the first and last rows."""
     import torch
-    M, N, K = 2047, 10256, 256
+    M, N = 2047, 10256
     W = F.synth_weight(qtype, N, K, seed=qtype)
-    aq, asc, absum = acts(qm, F.synth_activations(M, K, seed=3, outlier_frac=0.01), dev, M_stride=2048)
+    x = F.synth_activations(M, K, seed=3, outlier_frac=0.01)
+    aq, asc, absum = qm.quantize_act(to_dev(x, dev), M_stride=2048, act32=act32)
     w = qm.QWeight(qtype, to_dev(W, dev), N, K)
-    C = qm.gemm(w, aq, asc, absum, M=M).cpu().numpy()
+    C = qm.gemm(w, aq, asc, absum, M=M, act32=act32)
+    g = torch.randn((M, N), device=dev)
+    add = qm.gemm(w, aq, asc, absum, M=M, C=g.clone(), ldc=N, accumulate=1, act32=act32)
+    mul = qm.gemm(w, aq, asc, absum, M=M, C=g.clone(), ldc=N, accumulate=2, act32=act32)
+    assert torch.equal(add, g + C)
+    assert torch.allclose(mul, torch.nn.functional.silu(g) * C, rtol=1e-5, atol=1e-6 * C.abs().max().item())
+    C = C.cpu().numpy()
     isum = qm.gemm_blocksums(w, aq, M=M)
     a = (aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy())
     for r in (slice(0, 32), slice(N - 32, N)):
-        ref, risum, _ = oracle.blockdot(qtype, W[r], K, *a, M=M, blocksums=True)
+        if act32:
+            ref, risum, _ = oracle.blockdot(qtype, W[r], K, *a, M=M, blocksums=True)
+            assert np.array_equal(isum[:, r].cpu().numpy(), risum)
+        else:
+            ref = oracle.blockdot256(qtype, W[r], K, *a, M=M)
         assert rel_err(C[:, r], ref) < TOL_INT8_PATH
         assert_elementwise(C[:, r], ref)
-        assert np.array_equal(isum[:, r].cpu().numpy(), risum)

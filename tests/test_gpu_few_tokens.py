@@ -85,3 +85,16 @@ def test_long_rows_lose_no_precision(qm, dev, qtype):
     got = qm.gemv(w, aq, asc, absum, T=T).cpu().numpy().astype(np.float64)
     ref = oracle.blockdot(qtype, W, K, aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy(), M=T).astype(np.float64)
     assert np.sqrt(np.mean((got - ref) ** 2) / np.mean(ref ** 2)) < 1e-7
+
+
+@pytest.mark.parametrize("qtype", GEMV_TYPES)
+@pytest.mark.parametrize("N,K,M", [(48, 768, 5), (4112, 1280, 16), (48, 1280, 17), (8208, 1280, 16), (8208, 1280, 32)])
+def test_prompt_scales_per_256(qm, dev, qtype, N, K, M):
+    """Per-256 activation scales (one scale row per eight blocks), on each of the kernels and both token tiles."""
+    W = F.synth_weight(qtype, N, K, seed=qtype + N)
+    aq, asc, absum = qm.quantize_act(to_dev(F.synth_activations(M, K, seed=M, outlier_frac=0.01), dev), M_stride=M, act32=False)
+    w = qm.QWeight(qtype, to_dev(W, dev), N, K)
+    got = qm.gemm(w, aq, asc, absum, M=M, act32=False).cpu().numpy()
+    ref = oracle.blockdot256(qtype, W, K, aq.cpu().numpy(), asc.cpu().numpy(), absum.cpu().numpy(), M=M)
+    assert rel_err(got, ref) < TOL_INT8_PATH
+    assert_elementwise(got, ref)
