@@ -15,7 +15,7 @@ template <int TYPE, int NT>
 __device__ __forceinline__ void few_gateup(const GemmArgs& a, const typename LdsFor<TYPE>::type* tab,
                                            float (*part)[4 * 2 * 4][64], int e, int m0, int nvalid) {
   using Tr = Traits<TYPE>;
-  constexpr int W = 4, PF = TYPE == T_Q6_K ? 1 : 2;  // (Q6_K: a second stage spills)
+  constexpr int W = 4, PF = TYPE == T_Q6_K ? 1 : 2;  // (Q6_K spills 56 bytes with one stage, more with two)
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int K = a.w.K, nb = K / 32, nq = K / 128;
